@@ -311,6 +311,38 @@ void launch_xpass_ct(const Grid& g, const XBatch<T>& b, const T* bx, const T* by
                        b, g.tw<T>(0), bx, by, bz);
 }
 
+// two-stage kernels: LDS limits, and their launches
+template <typename T>
+void set_lds_attributes_two() {
+    static bool done = false;
+    if (done) return;
+    allow_lds(&slab_two_kernel<T>);
+    allow_lds(&pencil_two_kernel<T>);
+    allow_lds(&flat_steps_kernel<T, true>);
+    allow_lds(&flat_steps_kernel<T, false>);
+    done = true;
+}
+
+template <typename T>
+void launch_slab_two(const Grid& g, int mode, const SlabBatch<T>& b) {
+    // the first half step of a Richardson pair waits in the output slice
+    for (int i = 0; i < b.n; i++)
+        if (mode == SLAB_INV2 && !b.it[i].qout) throw Error("slab item without the real slice its second pass reads");
+    const TwoGeom& t = g.two[prec_index<T>()];
+    hipLaunchKernelGGL((slab_two_kernel<T>), dim3(g.tnx[0], b.n), dim3(two_slab_threads(t)),
+                       two_slab_lds(t, sizeof(typename vec2<T>::type)), g.stream(), t, mode, b, g.tw<T>(1),
+                       g.tw<T>(2));
+}
+
+template <typename T>
+void launch_xpass_two(const Grid& g, const XBatch<T>& b, const T* bx, const T* by, const T* bz) {
+    const TwoGeom& t = g.two[prec_index<T>()];
+    constexpr int e = sizeof(typename vec2<T>::type);
+    const int tiles = ceil_div(t.nzc, two_pencil_columns(e));
+    hipLaunchKernelGGL((pencil_two_kernel<T>), dim3(g.tnx[1] * tiles, b.n), dim3(64), two_pencil_lds(t, e), g.stream(),
+                       t, b, g.tw<T>(0), bx, by, bz);
+}
+
 template <typename T, int MODE, int MAXR, bool BIG>
 void launch_slab_k(const Grid& g, const SlabBatch<T>& b, dim3 grid, dim3 block, size_t lds) {
     hipLaunchKernelGGL((slab_kernel<T, MODE, MAXR, BIG>), grid, block, lds, g.stream(), g.sg, b, g.tw<T>(1),
@@ -451,6 +483,25 @@ void Grid::setup_fft() {
         Ms = (size_t)tnx[0] * tnx[1] * std::max(spitch, spitch32);
         tune_fft_schedule<double>();
         tune_fft_schedule<float>();
+    }
+    if (ct_n == 0) {
+        // Every other grid takes the two-stage kernels when its lengths have such a plan and a plane
+        // fits the LDS: a whole evaluation with them against the runtime-radix kernels of fts_fft.hpp
+        // (which keep lengths like 125, 17 k or above 256) measured 9.1 against 38.0 ms at 48x84x60
+        // (radix 7: those kernels run it from LDS twiddles and spill), 2.19 against 4.40 ms at
+        // 72x120x75 in FP32, 6.5 against 30.0 ms at 60x104 and 3.0 against 5.0 ms at 128 points in 1D.
+        // FP32 kernels carry no radix with a prime factor above 5, and big grids are refused in FP32
+        two_stage[0] = two_geometry(tnx, sizeof(double2), LDS_LIMIT, two[0]);
+        two_stage[1] = !big && two_geometry(tnx, sizeof(float2), LDS_LIMIT, two[1]);
+        if (two_stage[0]) {
+            spitch = two[0].sp;
+            set_lds_attributes_two<double>();
+        }
+        if (two_stage[1]) {
+            spitch32 = two[1].sp;
+            set_lds_attributes_two<float>();
+        }
+        Ms = (size_t)tnx[0] * tnx[1] * std::max(spitch, spitch32);
     }
 }
 
@@ -734,6 +785,10 @@ void Grid::launch_slab(int mode, const SlabBatch<T>& b) const {
         case 96: launch_slab_ct<T, 96>(*this, mode, b); break;
         case 128: launch_slab_ct<T, 128>(*this, mode, b); break;
         default: {
+            if (two_stage[prec_index<T>()]) {
+                launch_slab_two<T>(*this, mode, b);
+                break;
+            }
             const dim3 grid(tnx[0], b.n), block(slab_threads);
             const size_t lds = slab_lds<T>();
             if (mode == SLAB_FWD) launch_slab_mode<T, SLAB_FWD>(*this, b, grid, block, lds);
@@ -749,6 +804,7 @@ template <typename T>
 void Grid::launch_xpass(const XBatch<T>& b, const T* bx, const T* by, const T* bz) const {
     require_supported<T>(*this);
     if (b.n == 0) return;
+    if (tnx[0] == 1 && bx == nullptr) return;   // a transform of length 1
     KernelTimer& timer = ctx->timer;
     hipEvent_t start = timer.begin(stream(), FTS_KERNEL_PENCIL);
     switch (ct_n) {
@@ -758,6 +814,10 @@ void Grid::launch_xpass(const XBatch<T>& b, const T* bx, const T* by, const T* b
         case 96: launch_xpass_ct<T, 96>(*this, b, bx, by, bz); break;
         case 128: launch_xpass_ct<T, 128>(*this, b, bx, by, bz); break;
         default: {
+            if (two_stage[prec_index<T>()]) {
+                launch_xpass_two<T>(*this, b, bx, by, bz);
+                break;
+            }
             const dim3 grid(tnx[1] * xg.n_tiles, b.n), block(x_threads);
             if (big)
                 hipLaunchKernelGGL((xpass_kernel<T, true>), grid, block, x_lds<T>(), stream(), xg, b, tw<T>(0), bx,
@@ -770,6 +830,29 @@ void Grid::launch_xpass(const XBatch<T>& b, const T* bx, const T* by, const T* b
     FTS_HIP_CHECK(hipGetLastError());
     // each spectrum read and written once
     if (start) timer.end(stream(), start, FTS_KERNEL_PENCIL, 4.0 * sizeof(T) * Mc * b.n);
+}
+
+template <typename T>
+void Grid::launch_flat(bool continuous, const FlatBatch<T>& b, const T* by, const T* bz) const {
+    require_supported<T>(*this);
+    if (b.n == 0) return;
+    FTS_REQUIRE(flat<T>(), "flat steps need a grid of one x-slab with a two-stage plan");
+    const TwoGeom& t = two[prec_index<T>()];
+    const dim3 grid(b.n), block(two_slab_threads(t));
+    const size_t lds = two_slab_lds(t, sizeof(typename vec2<T>::type));
+    KernelTimer& timer = ctx->timer;
+    hipEvent_t start = timer.begin(stream(), FTS_KERNEL_SLAB);
+    if (continuous)
+        hipLaunchKernelGGL((flat_steps_kernel<T, true>), grid, block, lds, stream(), t, b, tw<T>(1), tw<T>(2), by, bz);
+    else
+        hipLaunchKernelGGL((flat_steps_kernel<T, false>), grid, block, lds, stream(), t, b, tw<T>(1), tw<T>(2), by, bz);
+    FTS_HIP_CHECK(hipGetLastError());
+    if (start) {
+        // each step writes its slice once; the first slice, w and the mask are read once
+        double bytes = 0.0;
+        for (int i = 0; i < b.n; i++) bytes += (double)sizeof(T) * M * (b.it[i].steps + 2 + (b.it[i].mask ? 1 : 0));
+        timer.end(stream(), start, FTS_KERNEL_SLAB, bytes);
+    }
 }
 
 template <typename T>
@@ -962,6 +1045,8 @@ template void Grid::launch_slab<double>(int, const SlabBatch<double>&) const;
 template void Grid::launch_slab<float>(int, const SlabBatch<float>&) const;
 template void Grid::launch_xpass<double>(const XBatch<double>&, const double*, const double*, const double*) const;
 template void Grid::launch_xpass<float>(const XBatch<float>&, const float*, const float*, const float*) const;
+template void Grid::launch_flat<double>(bool, const FlatBatch<double>&, const double*, const double*) const;
+template void Grid::launch_flat<float>(bool, const FlatBatch<float>&, const float*, const float*) const;
 template int Grid::launch_stress_pencil<double>(const StressBatch<double>&, const StressGeom&, const double*,
                                                 const double*, const double*, double*) const;
 template int Grid::launch_stress_pencil<float>(const StressBatch<float>&, const StressGeom&, const float*,

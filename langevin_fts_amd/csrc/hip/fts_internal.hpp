@@ -10,6 +10,7 @@
 #include "fts_common.hpp"
 #include "fts_fft.hpp"
 #include "fts_fft_ct.hpp"
+#include "fts_fft_two.hpp"
 #include "fts_fft_wl.hpp"
 
 namespace fts {
@@ -76,6 +77,7 @@ struct DotBatch {
 static_assert(sizeof(SlabBatch<double>) <= 4000, "slab batch exceeds the kernel-argument budget");
 static_assert(sizeof(XBatch<double>) <= 4000, "pencil batch exceeds the kernel-argument budget");
 static_assert(sizeof(DotBatch<double>) <= 4000, "dot batch exceeds the kernel-argument budget");
+static_assert(sizeof(FlatBatch<double>) <= 4000, "flat-step batch exceeds the kernel-argument budget");
 
 template <typename T>
 struct StressBatch;
@@ -112,6 +114,9 @@ public:
     bool big = false;        // some axis needs a radix outside {2, 3, 4, 5, 8}
     int ct_n = 0;        // N of the compile-time specialised kernels for an N^3 grid, 0: runtime kernels
     bool wave_local = false; // N^3 grids: one wavefront per line transform
+    // other grids whose lengths all have a two-stage plan, per precision ([0] FP64, [1] FP32)
+    bool two_stage[2] = {false, false};
+    TwoGeom two[2];
     // launch shapes of the wave-local kernels per precision ([0] FP64, [1] FP32):
     // slab workgroup size and pencil kz columns per wavefront, with how they were chosen
     int slab_bd[2] = {0, 0};
@@ -154,6 +159,13 @@ public:
     void launch_slab(int mode, const SlabBatch<T>& b) const;
     template <typename T>
     void launch_xpass(const XBatch<T>& b, const T* bx, const T* by, const T* bz) const;
+    // Grids of one x-slab with a two-stage plan: whole runs of steps in one launch. by, bz: bond tables.
+    template <typename T>
+    bool flat() const {
+        return tnx[0] == 1 && two_stage[sizeof(T) == sizeof(float) ? 1 : 0];
+    }
+    template <typename T>
+    void launch_flat(bool continuous, const FlatBatch<T>& b, const T* by, const T* bz) const;
     // The stress of b.n terms from the slab pass's output spectra, with their x transforms
     // fused into the reduction (wave-local grids only): 3 partial sums per workgroup into
     // partials, term-major; returns the workgroups per term.

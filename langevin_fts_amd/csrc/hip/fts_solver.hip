@@ -76,7 +76,7 @@ private:
         double bsq, weight;
         int table, block;
     };
-    enum { L_INIT, L_SLAB_FWD, L_SLAB_INV1, L_SLAB_INV2, L_XPASS, L_REAL };
+    enum { L_INIT, L_SLAB_FWD, L_SLAB_INV1, L_SLAB_INV2, L_XPASS, L_REAL, L_FLAT };
     struct Launch {
         int type, idx;
     };
@@ -103,6 +103,7 @@ private:
     void emit_x(const std::vector<XItem<T>>& items);
     void emit_init(const std::vector<InitItem<T>>& items);
     void emit_real(const std::vector<RealItem>& items);
+    void emit_flat(const std::vector<FlatItem<T>>& items);
     void build_real_tables();
     void launch_real(const RealBatch& b);
     void build_slice(const std::vector<std::array<int, 3>>& jobs);
@@ -156,6 +157,7 @@ private:
     std::vector<InitBatch<T>> inits_;
     std::vector<SlabBatch<T>> slabs_;
     std::vector<XBatch<T>> xs_;
+    std::vector<FlatBatch<T>> flats_;
     // real-space Crank-Nicolson form
     bool real_ = false;
     bool real_plain_ = false;   // env FTS_REAL_PLAIN_SWEEPS=1: one thread per line on every axis
@@ -354,6 +356,18 @@ void Solver<T>::emit_real(const std::vector<RealItem>& items) {
         for (int k = 0; k < b.n; k++) b.it[k] = items[i + k];
         launches_.push_back({L_REAL, (int)reals_.size()});
         reals_.push_back(b);
+    }
+}
+
+template <typename T>
+void Solver<T>::emit_flat(const std::vector<FlatItem<T>>& items) {
+    for (size_t i = 0; i < items.size(); i += FLAT_BATCH) {
+        FlatBatch<T> b{};
+        b.n = (int)std::min<size_t>(FLAT_BATCH, items.size() - i);
+        b.stride = (size_t)M_;
+        for (int k = 0; k < b.n; k++) b.it[k] = items[i + k];
+        launches_.push_back({L_FLAT, (int)flats_.size()});
+        flats_.push_back(b);
     }
 }
 
@@ -617,7 +631,27 @@ void Solver<T>::build_slice(const std::vector<std::array<int, 3>>& jobs) {
         runs.push_back({p, (int)s, n0, cnt});
         D = std::max(D, cnt);
     }
-    for (int t = 0; t < D; t++) {
+    // grids of one x-slab: a run's steps need nothing of the other runs, one launch for all of them
+    const bool flat = !real_ && g_->template flat<T>();
+    if (flat) {
+        std::vector<FlatItem<T>> items;
+        for (auto& r : runs) {
+            const int m = props_[r.p].monomer;
+            FlatItem<T> it{};
+            it.q = q(r.p, r.n0);
+            it.half = reinterpret_cast<T*>(slot(2 * r.slot));
+            it.w = model_ == FTS_CONTINUOUS ? w(m) : ew(m);
+            it.mask = mask();
+            it.full_w = model_ == FTS_CONTINUOUS ? ds / 2 : ew_coef();
+            it.half_w = ds / 4;
+            it.steps = r.cnt;
+            it.full_table = full(m);
+            it.half_table = half(m);
+            items.push_back(it);
+        }
+        emit_flat(items);
+    }
+    for (int t = 0; t < D && !flat; t++) {
         std::vector<SlabItem<T>> fw, inv1, inv2;
         std::vector<XItem<T>> x1, x2;
         std::vector<RealItem> ri;
@@ -819,6 +853,7 @@ void Solver<T>::run_launches() {
             case L_SLAB_INV2: g_->launch_slab<T>(SLAB_INV2, slabs_[L.idx]); break;
             case L_XPASS: g_->launch_xpass<T>(xs_[L.idx], bx, by, bz); break;
             case L_REAL: launch_real(reals_[L.idx]); break;
+            case L_FLAT: g_->template launch_flat<T>(model_ == FTS_CONTINUOUS, flats_[L.idx], by, bz); break;
         }
     }
 }

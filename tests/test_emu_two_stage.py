@@ -1,0 +1,111 @@
+"""The two-stage FFT kernels of fts_fft_two.hpp, built for the host from their own source by
+tests/emu/fft_two_emu.cpp and run as emulated workgroups with AddressSanitizer on the LDS block
+and on every global buffer (NaN in what was never written): forward and inverse transforms
+against numpy, a convolution with the bond factors, and two masked propagator steps of each kind
+by the slab and pencil passes and by the one-launch kernel of flat grids, against numpy in FP64.
+The grids take every radix 1..16 on the axes, odd and even lengths (rows without a partner, no
+Nyquist column), more butterflies than threads, and the plans' limits. CPU only.
+
+Tolerances: a transform's rounding error grows as eps log2(M) in the 2-norm; 64 eps bounds each
+result's largest error over its largest value for the steps' 12 transforms at these sizes."""
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+EMU = os.path.join(REPO, "tests", "emu")
+HIP = os.path.join(REPO, "langevin_fts_amd", "csrc", "hip")
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None or not os.path.isdir(EMU),
+                                reason="needs g++ and tests/emu")
+
+
+@pytest.fixture(scope="module")
+def exe(tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("emu") / "fft_two_emu")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fsanitize=address", "-fno-omit-frame-pointer", "-I", EMU,
+                    "-I", HIP, "-o", path, os.path.join(EMU, "fft_two_emu.cpp")], check=True, capture_output=True)
+    return path
+
+
+def run(exe, op, esize, n, a, tmp):
+    fi, fo = os.path.join(tmp, "in.bin"), os.path.join(tmp, "out.bin")
+    dt = np.float32 if esize == 4 else np.float64
+    np.ascontiguousarray(a, dtype=dt).tofile(fi)
+    r = subprocess.run([exe, op, str(esize)] + [str(x) for x in n] + [fi, fo], capture_output=True, text=True,
+                       timeout=600, env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
+    assert r.returncode == 0, r.stdout + r.stderr
+    return np.fromfile(fo, dtype=dt).astype(np.float64)
+
+
+def bond(n, share):
+    f = 1.0
+    for d, L in enumerate(n):
+        k = np.arange(L // 2 + 1 if d == 2 else L)
+        k = np.minimum(k, L - k)
+        f = f * np.exp(-0.3 * share * (k / L) ** 2).reshape([-1 if i == d else 1 for i in range(3)])
+    return f
+
+
+def conv(n, q, share):
+    return np.fft.irfftn(bond(n, share) * np.fft.rfftn(q), s=n, axes=(0, 1, 2))
+
+
+def off(x, y):
+    return float(np.max(np.abs(x - y.ravel())) / np.max(np.abs(y)))
+
+
+def check(exe, n, esize, ops, tmp):
+    rng = np.random.default_rng(sum(n))
+    q, w = 1.0 + 0.3 * rng.standard_normal(n), rng.standard_normal(n)
+    mask = (rng.random(n) > 0.2).astype(np.float64)
+    if esize == 4:
+        q, w = q.astype(np.float32).astype(np.float64), w.astype(np.float32).astype(np.float64)
+    tol = 64 * (2.0 ** -53 if esize == 8 else 2.0 ** -24)
+    ds = 0.25
+    for op in ops:
+        if op == "fft":
+            ref = np.fft.rfftn(q)
+            got = run(exe, op, esize, n, q, tmp)
+            e = off(got, np.stack([ref.real, ref.imag], -1))
+        elif op == "ifft":
+            ref = np.fft.rfftn(q)
+            e = off(run(exe, op, esize, n, np.stack([ref.real, ref.imag], -1), tmp), q)
+        elif op == "conv":
+            e = off(run(exe, op, esize, n, q, tmp), conv(n, q, 1.0))
+        else:
+            out, x = [], q
+            for _ in range(2):
+                if op == "flatd":
+                    x = np.exp(-w * ds) * conv(n, x, 1.0) * mask
+                else:
+                    e2, e4 = np.exp(-w * ds / 2), np.exp(-w * ds / 4)
+                    q1 = e2 * conv(n, e2 * x, 1.0)
+                    q2 = e4 * conv(n, e2 * conv(n, e4 * x, 0.5), 0.5)
+                    x = (4 * q2 - q1) / 3 * mask
+                out.append(x)
+            got = run(exe, op, esize, n, np.concatenate([q.ravel(), w.ravel(), mask.ravel()]), tmp)
+            e = off(got, np.stack(out))
+        print(n, esize, op, f"{e:.1e}", flush=True)
+        assert e < tol, (n, esize, op, e)
+
+
+# (x, y, z): every radix as r1 and as r2 of a y and of a z plan, odd and even lengths
+GRIDS = [(2, 8, 8), (3, 6, 10), (4, 12, 9), (5, 15, 16), (7, 14, 26), (11, 22, 33), (13, 21, 35), (2, 45, 20),
+         (6, 7, 13), (1, 60, 104), (1, 1, 128), (1, 1, 30), (2, 30, 27), (9, 10, 1), (16, 3, 4), (2, 49, 25),
+         (1, 9, 11), (3, 1, 24)]
+
+
+@pytest.mark.parametrize("n", GRIDS)
+def test_two_stage_fp64(exe, n, tmp_path):
+    ops = ["fft", "ifft", "conv", "step"] + (["flat", "flatd"] if n[0] == 1 else [])
+    check(exe, n, 8, ops, str(tmp_path))
+
+
+@pytest.mark.parametrize("n", [(2, 8, 8), (3, 6, 10), (5, 15, 16), (1, 20, 48), (1, 1, 128)])
+def test_two_stage_fp32(exe, n, tmp_path):
+    ops = ["fft", "ifft", "conv", "step"] + (["flat", "flatd"] if n[0] == 1 else [])
+    check(exe, n, 4, ops, str(tmp_path))

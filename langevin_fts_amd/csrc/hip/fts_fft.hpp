@@ -303,10 +303,10 @@ struct SlabItem {
     T* qout;           // real output of the inverse part (nullptr: no write)
     typename vec2<T>::type* c0;
     typename vec2<T>::type* c1;
-    const T* w;        // field for exp(-w*coef) factors (nullptr: all factors 1; coef < 0: w is the factor)
+    const T* w;        // factor table, see factor(); nullptr: all factors 1
     const T* mask;     // nullptr: no mask
-    T post0, post1;    // inverse part: r_o *= exp(-w*post_o) / M
-    T pre0, pre1;      // forward part: spectrum_o = FFT[exp(-w*pre_o) q]
+    T post0, post1;    // inverse part: r_o *= factor(post_o) / M
+    T pre0, pre1;      // forward part: spectrum_o = FFT[factor(pre_o) q]
     int n_out;         // FWD mode: 1 or 2 spectra
     int forward;       // INV modes: continue with the forward part
 };
@@ -318,13 +318,6 @@ struct SlabBatch {
 };
 
 enum SlabMode { SLAB_FWD = 0, SLAB_INV1 = 1, SLAB_INV2 = 2 };
-
-template <typename T>
-__device__ __forceinline__ T fexp(T x);
-template <>
-__device__ __forceinline__ double fexp<double>(double x) { return exp(x); }
-template <>
-__device__ __forceinline__ float fexp<float>(float x) { return __expf(x); }
 
 // In LDS the pair of rows (2p, 2p+1) of a slab is packed as one complex row of
 // length nz starting at S[2p*P]: row 2p in .x, row 2p+1 in .y. Each thread owns
@@ -439,10 +432,13 @@ __device__ __forceinline__ void store_spectrum(const T2* S, const SlabGeom& g, T
     }
 }
 
+// The step factor of a point, from a table of exponentials made once per call: FACTOR_TABLE takes
+// the value as it is, FACTOR_SQUARE squared; coef 0 or no table: 1.
+constexpr double FACTOR_TABLE = -1.0, FACTOR_SQUARE = -2.0;
 template <typename T>
 __device__ __forceinline__ T factor(T w, bool has_w, T coef) {
-    // coef < 0: the array already holds the factor exp(-w ds) (a table made once per call)
-    return (has_w && coef != (T)0) ? (coef < (T)0 ? w : fexp<T>(-w * coef)) : (T)1;
+    if (!has_w || coef == (T)0) return (T)1;
+    return coef == (T)FACTOR_SQUARE ? w * w : w;
 }
 
 // write this thread's real values times exp(-w*coef) into the packed rows

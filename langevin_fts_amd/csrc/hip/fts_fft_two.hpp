@@ -22,7 +22,7 @@
 
 #include <type_traits>
 
-#include "fts_fft.hpp"
+#include "fts_two_plan.hpp"
 
 namespace fts {
 
@@ -210,118 +210,11 @@ struct RDft<11, DIR, T, T2> : RDftPrime<11, DIR, T, T2> {};
 template <int DIR, typename T, typename T2>
 struct RDft<13, DIR, T, T2> : RDftPrime<13, DIR, T, T2> {};
 
-// ------------------------------------------------------------------ plans
-constexpr int TWO_MAXR = 16;
-
-// radices the kernels of a precision are built with (FP32 plans take prime factors 2, 3 and 5 only)
-constexpr bool two_radix(int r, bool fp32) {
-    return r >= 1 && r <= TWO_MAXR && !(fp32 && (r % 7 == 0 || r % 11 == 0 || r % 13 == 0));
-}
-
-struct TwoAxis {
-    int L, r1, r2;
-};
-
-// L = r1 r2 with the smallest larger radix. y axis: r1 even when L is (rows pair up inside a
-// butterfly), and the larger one when L is odd (one row of r1 has no partner). Other axes: the
-// larger radix is r2, the run of consecutive z values that a wavefront stores.
-inline bool two_axis(int L, bool y_axis, bool fp32, TwoAxis& a) {
-    a = TwoAxis{L, 0, 0};
-    for (int m = 1; m <= TWO_MAXR && !a.r1; m++)
-        for (int s = 1; s <= m && !a.r1; s++) {
-            if (m * s != L || !two_radix(m, fp32) || !two_radix(s, fp32)) continue;
-            const bool first_large = y_axis && (L % 2 == 1 || s % 2 == 1);
-            a.r1 = first_large ? m : s;
-            a.r2 = first_large ? s : m;
-        }
-    return a.r1 != 0;
-}
-
-struct TwoGeom {
-    int nx, nzc, sp;      // x-slabs, half-spectrum columns and their row pitch
-    TwoAxis x, y, z;
-    int lines;            // packed z lines: ceil(y.r1 / 2) y.r2
-    int pad;              // one pad slot after every z.r1 positions of a line (z.r1 even), else 0
-    int pitch;            // slots of a line
-    int xpad;             // pencil pass: extra slots between the stage-B groups
-    unsigned m_nzc, m_zr1, m_zr2, m_yr2;   // reciprocals for two_div
-    double inv_m;
-};
-
-// t / d for t d < 2^32 by one multiplication with m = two_recip(d)
-constexpr unsigned two_recip(int d) { return d == 1 ? 0u : (unsigned)(((1ull << 32) + d - 1) / d); }
-__device__ __forceinline__ int two_div(int t, unsigned m) {
-    return m == 0 ? t : (int)(((unsigned long long)(unsigned)t * m) >> 32);
-}
-
-// Wavefront accesses of the two z stages that share an LDS bank, counted over groups of `row`
-// consecutive lanes (row: elements of one 256-byte bank row)
-inline int two_conflicts(const TwoGeom& g, int pitch, int row) {
-    int total = 0;
-    for (int stage = 0; stage < 2; stage++) {
-        const int r = stage == 0 ? g.z.r1 : g.z.r2, step = stage == 0 ? 1 : g.z.r1 + g.pad;
-        for (int t0 = 0; t0 < 64; t0 += row) {
-            int hit[64] = {}, worst = 0;
-            for (int t = t0; t < t0 + row; t++) {
-                const int b = ((t / r) * pitch + (t % r) * step) % row;
-                worst = std::max(worst, ++hit[b]);
-            }
-            total += worst;
-        }
-    }
-    return total;
-}
-
-// The geometry of an nx x ny x nz grid, or false when a length has no plan or a plane does not
-// fit the LDS
-inline bool two_geometry(const int* n, int elem_bytes, size_t lds_limit, TwoGeom& g) {
-    g = TwoGeom{};
-    const bool fp32 = elem_bytes == 8;
-    if (!two_axis(n[0], false, fp32, g.x) || !two_axis(n[1], true, fp32, g.y) || !two_axis(n[2], false, fp32, g.z))
-        return false;
-    g.nx = n[0];
-    g.nzc = n[2] / 2 + 1;
-    const int line = 128 / elem_bytes;
-    g.sp = (g.nzc + line - 1) / line * line;
-    g.lines = (g.y.r1 + 1) / 2 * g.y.r2;
-    g.pad = g.z.r1 % 2 == 0 ? 1 : 0;
-    const int row = 256 / elem_bytes, least = n[2] + g.pad * g.z.r2 + 2;
-    int best = 1 << 30;
-    for (int p = least; p < least + row; p++) {
-        const int c = two_conflicts(g, p, row);
-        if (c < best) {
-            best = c;
-            g.pitch = p;
-        }
-    }
-    auto bytes = [&] { return (size_t)(g.lines * g.pitch + n[1] + n[2]) * elem_bytes; };
-    if (bytes() > lds_limit) g.pitch = least;
-    if (bytes() > lds_limit) return false;
-    // pencil pass: groups of r2 rows of a tile's `line` columns, started line columns apart (mod the bank row)
-    g.xpad = (line - g.x.r2 * line % row + row) % row;
-    g.m_nzc = two_recip(g.nzc);
-    g.m_zr1 = two_recip(g.z.r1);
-    g.m_zr2 = two_recip(g.z.r2);
-    g.m_yr2 = two_recip(g.y.r2);
-    g.inv_m = 1.0 / ((double)n[0] * n[1] * n[2]);
-    return true;
-}
-inline size_t two_slab_lds(const TwoGeom& g, int elem_bytes) {
-    return (size_t)(g.lines * g.pitch + g.y.L + g.z.L) * elem_bytes;
-}
-inline int two_pencil_columns(int elem_bytes) { return 128 / elem_bytes; }
-inline size_t two_pencil_lds(const TwoGeom& g, int elem_bytes) {
-    const int C = two_pencil_columns(elem_bytes);
-    return (size_t)(g.x.r1 * (g.x.r2 * C + g.xpad) + g.x.L) * elem_bytes;
-}
-// threads of a slab workgroup: one butterfly of the busiest stage each, at most TWO_BD
-constexpr int TWO_BD = 512;
-inline int two_slab_threads(const TwoGeom& g) {
-    const int y = g.nzc * std::max(g.y.r1, g.y.r2), z = g.lines * std::max(g.z.r1, g.z.r2);
-    return std::min(TWO_BD, (std::max(y, z) + 63) / 64 * 64);
-}
-
 // f with a compile-time radix equal to r
+template <typename T, typename F, int R>
+__device__ __forceinline__ void two_radix_call(std::integral_constant<int, R> r, F&& f) {
+    f(r);
+}
 template <typename T, typename F>
 __device__ __forceinline__ void two_radix_call(int r, F&& f) {
     constexpr bool fp64 = std::is_same<T, double>::value;
@@ -352,10 +245,10 @@ __device__ __forceinline__ void two_radix_call(int r, F&& f) {
 }
 
 // ------------------------------------------------------------------ the plane of a slab
-template <typename T>
+template <typename T, typename G>
 struct TwoPlane {
     using T2 = typename vec2<T>::type;
-    const TwoGeom& g;
+    G g;
     T2* S;            // packed lines
     const T2 *Wy, *Wz;
     int tid, bd;
@@ -367,7 +260,7 @@ struct TwoPlane {
     };
     __device__ __forceinline__ int zslot(int k) const { return g.pad ? k + two_div(k, g.m_zr1) : k; }
     __device__ __forceinline__ Col column(int c) const {
-        const int nz = g.z.L, end = nz + g.pad * g.z.r2;
+        const int nz = g.z.L, end = nz + g.pad * g.zr2;
         if (c == 0) return Col{0, end, true};
         if (2 * c == nz) return Col{zslot(c), end + 1, true};
         return Col{zslot(c), zslot(nz - c), false};
@@ -377,21 +270,21 @@ struct TwoPlane {
     template <int R>
     __device__ __forceinline__ void y_scatter(T2 (&v)[R], const Col& q, int j) const {
         RDft<R, +1, T, T2>::run(v);
-        T2* base = S + (j >> 1) * g.y.r2 * g.pitch + ((j & 1) ? q.o : q.e);
+        T2* base = S + (j >> 1) * g.yr2 * g.pitch + ((j & 1) ? q.o : q.e);
 #pragma unroll
         for (int r = 0; r < R; r++) base[r * g.pitch] = v[r];
     }
     // stage A of y, inverse, with the merge of the row pairs
     __device__ __forceinline__ void y_merge() const {
-        const int total = g.nzc * g.y.r2;
+        const int total = g.nzc * g.yr2;
         for (int t = tid; t < total; t += bd) {
             const int j = two_div(t, g.m_nzc), c = t - j * g.nzc;
             const Col q = column(c);
-            two_radix_call<T>(g.y.r1, [&](auto RC) {
+            two_radix_call<T>(g.yr1, [&](auto RC) {
                 constexpr int R = decltype(RC)::value;
                 T2 v[R];
 #pragma unroll
-                for (int r = 0; r < R; r++) v[r] = S[((r >> 1) * g.y.r2 + j) * g.pitch + ((r & 1) ? q.o : q.e)];
+                for (int r = 0; r < R; r++) v[r] = S[((r >> 1) * g.yr2 + j) * g.pitch + ((r & 1) ? q.o : q.e)];
 #pragma unroll
                 for (int r = 1; r < R; r++) v[r] = cmul(v[r], root<+1>(Wy, r * j));
                 RDft<R, +1, T, T2>::run(v);
@@ -399,7 +292,7 @@ struct TwoPlane {
                 for (int a = 0; a < (R + 1) / 2; a++) {
                     T2 A = v[2 * a], B = 2 * a + 1 < R ? v[(2 * a + 1) % R] : T2{(T)0, (T)0};
                     if (q.self) A.y = B.y = (T)0;
-                    T2* base = S + (a * g.y.r2 + j) * g.pitch;
+                    T2* base = S + (a * g.yr2 + j) * g.pitch;
                     base[q.e] = T2{A.x - B.y, A.y + B.x};
                     if (!q.self) base[q.o] = T2{A.x + B.y, B.x - A.y};
                 }
@@ -409,11 +302,11 @@ struct TwoPlane {
     // stage B of z: inverse (k natural -> (k1, n2)) or forward ((k1, n2) -> k natural)
     template <int DIR>
     __device__ __forceinline__ void z_outer() const {
-        const int total = g.lines * g.z.r1, step = g.z.r1 + g.pad;
+        const int total = g.lines * g.zr1, step = g.zr1 + g.pad;
         for (int t = tid; t < total; t += bd) {
-            const int line = two_div(t, g.m_zr1), j = t - line * g.z.r1;
+            const int line = two_div(t, g.m_zr1), j = t - line * g.zr1;
             T2* base = S + line * g.pitch + j;
-            two_radix_call<T>(g.z.r2, [&](auto RC) {
+            two_radix_call<T>(g.zr2, [&](auto RC) {
                 constexpr int R = decltype(RC)::value;
                 T2 v[R];
 #pragma unroll
@@ -429,16 +322,16 @@ struct TwoPlane {
     // values; it returns through them what the forward transform takes.
     template <typename Op>
     __device__ __forceinline__ void z_inner(bool inverse, bool forward, Op&& op) const {
-        const int total = g.lines * g.z.r2;
+        const int total = g.lines * g.zr2;
         const int nz = g.z.L;
         for (int t = tid; t < total; t += bd) {
-            const int line = two_div(t, g.m_zr2), j = t - line * g.z.r2;
+            const int line = two_div(t, g.m_zr2), j = t - line * g.zr2;
             const int a = two_div(line, g.m_yr2);
-            const int row = line + a * g.y.r2;    // (2 a) r2 + n2 with line = a r2 + n2
-            const bool two = 2 * a + 1 < g.y.r1;
+            const int row = line + a * g.yr2;    // (2 a) r2 + n2 with line = a r2 + n2
+            const bool two = 2 * a + 1 < g.yr1;
             const int i0 = row * nz + j;
-            T2* base = S + line * g.pitch + j * (g.z.r1 + g.pad);
-            two_radix_call<T>(g.z.r1, [&](auto RC) {
+            T2* base = S + line * g.pitch + j * (g.zr1 + g.pad);
+            two_radix_call<T>(g.zr1, [&](auto RC) {
                 constexpr int R = decltype(RC)::value;
                 T2 v[R];
                 if (inverse) {
@@ -449,7 +342,7 @@ struct TwoPlane {
                     RDft<R, +1, T, T2>::run(v);
                 }
 #pragma unroll
-                for (int r = 0; r < R; r++) op(i0 + r * g.z.r2, two, v[r]);
+                for (int r = 0; r < R; r++) op(i0 + r * g.zr2, two, v[r]);
                 if (forward) {
                     RDft<R, -1, T, T2>::run(v);
 #pragma unroll
@@ -463,16 +356,16 @@ struct TwoPlane {
     // stage A of y, forward, with the split of the packed lines (twice the rows' spectra: the
     // caller halves the real values)
     __device__ __forceinline__ void y_split() const {
-        const int total = g.nzc * g.y.r2;
+        const int total = g.nzc * g.yr2;
         for (int t = tid; t < total; t += bd) {
             const int j = two_div(t, g.m_nzc), c = t - j * g.nzc;
             const Col q = column(c);
-            two_radix_call<T>(g.y.r1, [&](auto RC) {
+            two_radix_call<T>(g.yr1, [&](auto RC) {
                 constexpr int R = decltype(RC)::value;
                 T2 v[R];
 #pragma unroll
                 for (int a = 0; a < (R + 1) / 2; a++) {
-                    const T2* base = S + (a * g.y.r2 + j) * g.pitch;
+                    const T2* base = S + (a * g.yr2 + j) * g.pitch;
                     const T2 A = base[q.e];
                     const T2 B = q.self ? A : base[q.o];
                     v[2 * a] = T2{A.x + B.x, A.y - B.y};
@@ -482,14 +375,14 @@ struct TwoPlane {
 #pragma unroll
                 for (int r = 1; r < R; r++) v[r] = cmul(v[r], root<-1>(Wy, r * j));
 #pragma unroll
-                for (int r = 0; r < R; r++) S[((r >> 1) * g.y.r2 + j) * g.pitch + ((r & 1) ? q.o : q.e)] = v[r];
+                for (int r = 0; r < R; r++) S[((r >> 1) * g.yr2 + j) * g.pitch + ((r & 1) ? q.o : q.e)] = v[r];
             });
         }
     }
     // stage B of y, forward: v[r] becomes row j + r1 r of the column
     template <int R>
     __device__ __forceinline__ void y_gather(T2 (&v)[R], const Col& q, int j) const {
-        const T2* base = S + (j >> 1) * g.y.r2 * g.pitch + ((j & 1) ? q.o : q.e);
+        const T2* base = S + (j >> 1) * g.yr2 * g.pitch + ((j & 1) ? q.o : q.e);
 #pragma unroll
         for (int r = 0; r < R; r++) v[r] = base[r * g.pitch];
         RDft<R, -1, T, T2>::run(v);
@@ -500,17 +393,17 @@ struct TwoPlane {
 // The pass of fts_fft.hpp's slab_kernel (same items, modes and results) for grids with a
 // TwoGeom; spectra have rows of g.sp values. INV2 items must have qout: the first half step
 // waits there.
-template <typename T>
-__global__ void __launch_bounds__(TWO_BD) slab_two_kernel(TwoGeom g, int mode, SlabBatch<T> batch,
-                                                          const typename vec2<T>::type* twy,
-                                                          const typename vec2<T>::type* twz) {
+template <typename T, typename G>
+__device__ __forceinline__ void slab_two(const G& g, int mode, int bd, const SlabBatch<T>& batch,
+                                         const typename vec2<T>::type* twy, const typename vec2<T>::type* twz) {
     using T2 = typename vec2<T>::type;
+    using Plane = TwoPlane<T, G>;
     FTS_DYNAMIC_LDS(smem_raw);
     T2* S = reinterpret_cast<T2*>(smem_raw);
     T2* Wy = S + g.lines * g.pitch;
     T2* Wz = Wy + g.y.L;
-    for (int m = threadIdx.x; m < g.y.L; m += blockDim.x) Wy[m] = twy[m];
-    for (int m = threadIdx.x; m < g.z.L; m += blockDim.x) Wz[m] = twz[m];
+    for (int m = threadIdx.x; m < g.y.L; m += bd) Wy[m] = twy[m];
+    for (int m = threadIdx.x; m < g.z.L; m += bd) Wz[m] = twz[m];
     const SlabItem<T>& it = batch.it[blockIdx.y];
     const int ny = g.y.L, nz = g.z.L;
     const size_t roff = (size_t)blockIdx.x * ny * nz;
@@ -520,8 +413,8 @@ __global__ void __launch_bounds__(TWO_BD) slab_two_kernel(TwoGeom g, int mode, S
     const T* w = has_w ? it.w + roff : nullptr;
     const T* mask = it.mask ? it.mask + roff : nullptr;
     T* qout = it.qout ? it.qout + roff : nullptr;
-    const int second = g.y.r2 * nz;   // from a value of a pair's first row to the second's
-    const TwoPlane<T> pl{g, S, Wy, Wz, (int)threadIdx.x, (int)blockDim.x};
+    const int second = g.yr2 * nz;   // from a value of a pair's first row to the second's
+    const Plane pl{g, S, Wy, Wz, (int)threadIdx.x, bd};
 
     // FWD: n_out forward transforms of qin. INV1: inverse, store, forward. INV2: the inverse of
     // the full step (parked in qout); that of the half steps, combined with it, and the first
@@ -537,16 +430,16 @@ __global__ void __launch_bounds__(TWO_BD) slab_two_kernel(TwoGeom g, int mode, S
         __syncthreads();   // twiddles stored; the previous use of the plane is over
         if (inverse) {
             const T2* spec = (comb ? it.c1 : it.c0) + coff;
-            const int total = g.nzc * g.y.r1;
+            const int total = g.nzc * g.yr1;
             for (int t = pl.tid; t < total; t += pl.bd) {
                 const int j = two_div(t, g.m_nzc), c = t - j * g.nzc;
-                const typename TwoPlane<T>::Col q = pl.column(c);
-                two_radix_call<T>(g.y.r2, [&](auto RC) {
+                const typename Plane::Col q = pl.column(c);
+                two_radix_call<T>(g.yr2, [&](auto RC) {
                     constexpr int R = decltype(RC)::value;
                     T2 v[R];
                     const T2* src = spec + (size_t)j * g.sp + c;
 #pragma unroll
-                    for (int r = 0; r < R; r++) v[r] = src[r * g.y.r1 * g.sp];
+                    for (int r = 0; r < R; r++) v[r] = src[r * g.yr1 * g.sp];
                     pl.template y_scatter<R>(v, q, j);
                 });
             }
@@ -582,24 +475,247 @@ __global__ void __launch_bounds__(TWO_BD) slab_two_kernel(TwoGeom g, int mode, S
         pl.y_split();
         __syncthreads();
         T2* spec = (out == 1 ? it.c1 : it.c0) + coff;
-        const int total = g.nzc * g.y.r1;
+        const int total = g.nzc * g.yr1;
         for (int t = pl.tid; t < total; t += pl.bd) {
             const int j = two_div(t, g.m_nzc), c = t - j * g.nzc;
-            const typename TwoPlane<T>::Col q = pl.column(c);
-            two_radix_call<T>(g.y.r2, [&](auto RC) {
+            const typename Plane::Col q = pl.column(c);
+            two_radix_call<T>(g.yr2, [&](auto RC) {
                 constexpr int R = decltype(RC)::value;
                 T2 v[R];
                 pl.template y_gather<R>(v, q, j);
                 T2* dst = spec + (size_t)j * g.sp + c;
 #pragma unroll
-                for (int r = 0; r < R; r++) dst[r * g.y.r1 * g.sp] = v[r];
+                for (int r = 0; r < R; r++) dst[r * g.yr1 * g.sp] = v[r];
             });
         }
     }
 }
 
+template <typename T>
+__global__ void __launch_bounds__(TWO_BD) slab_two_kernel(TwoGeom g, int mode, SlabBatch<T> batch,
+                                                          const typename vec2<T>::type* twy,
+                                                          const typename vec2<T>::type* twz) {
+    slab_two<T>(TwoView(g), mode, blockDim.x, batch, twy, twz);
+}
+// The same pass for an N^3 grid with the plan, the workgroup size and the number of butterflies
+// per thread as constants. The real values of a thread's z butterflies stay in registers from
+// the inverse to the last forward transform, and every global load is issued a phase or more before
+// its use: the first spectrum and w before the first barrier, the second spectrum of a
+// Richardson step when the first has left its registers.
+template <typename T, int N, int BD>
+struct CubeSlab {
+    using T2 = typename vec2<T>::type;
+    using G = TwoCube<N, sizeof(T2)>;
+    static constexpr int YT = (G::nzc * G::y.r1 + BD - 1) / BD;    // y stage B butterflies per thread
+    static constexpr int ZT = (G::lines * G::z.r2 + BD - 1) / BD;  // z stage A butterflies per thread
+    static constexpr int RY = G::y.r2, RZ = G::z.r1;
+    // w stays in registers for the whole kernel unless its values, the real values and a butterfly
+    // of the largest radix exceed the registers of BD threads
+    static constexpr int VGPRS = BD > 512 ? 128 : 256;
+    static constexpr int WORDS = sizeof(T) / 4;
+    static constexpr bool W_RESIDENT = WORDS * (2 * 2 * ZT * RZ + 2 * 16) <= VGPRS - 40;
+    // the second spectrum is loaded ahead when that many registers are left
+    static constexpr bool AHEAD = WORDS * (2 * 2 * ZT * RZ + 2 * YT * RY + 2 * 16) <= VGPRS - 40;
+};
+
+template <typename T, int MODE, int N, int BD>
+__global__ void __launch_bounds__(BD) slab_cube_kernel(SlabBatch<T> batch, const typename vec2<T>::type* twy,
+                                                       const typename vec2<T>::type* twz) {
+    using T2 = typename vec2<T>::type;
+    using K = CubeSlab<T, N, BD>;
+    using G = typename K::G;
+    using Plane = TwoPlane<T, G>;
+    constexpr int YT = K::YT, ZT = K::ZT, RY = K::RY, RZ = K::RZ;
+    constexpr int Y_TASKS = G::nzc * G::y.r1, Z_TASKS = G::lines * G::z.r2;
+    FTS_DYNAMIC_LDS(smem_raw);
+    T2* S = reinterpret_cast<T2*>(smem_raw);
+    T2* Wy = S + G::lines * G::pitch;
+    T2* Wz = Wy + N;
+    const int tid = threadIdx.x;
+    const SlabItem<T>& it = batch.it[blockIdx.y];
+    const size_t roff = (size_t)blockIdx.x * N * N, coff = (size_t)blockIdx.x * N * G::sp;
+    const T inv_m = (T)G::inv_m;
+    const bool has_w = it.w != nullptr;
+    constexpr G g{};
+    const Plane pl{g, S, Wy, Wz, tid, BD};
+    constexpr int SECOND = G::y.r2 * N;   // from a value of a pair's first row to the second's
+
+    // y stage B butterfly k of this thread: column and k1
+    auto y_task = [&](int k, int& c, int& j) {
+        const int t = tid + k * BD;
+        j = t / G::nzc;
+        c = t - j * G::nzc;
+        return Y_TASKS % BD == 0 || t < Y_TASKS;
+    };
+    auto fetch = [&](const T2* spec, T2 (&v)[YT][RY]) {
+#pragma unroll
+        for (int k = 0; k < YT; k++) {
+            int c, j;
+            if (y_task(k, c, j)) {
+#pragma unroll
+                for (int r = 0; r < RY; r++) v[k][r] = spec[(j + r * G::y.r1) * G::sp + c];
+            }
+        }
+    };
+    // z stage A butterfly k: its LDS values and the index of its first real value
+    auto z_task = [&](int k, int& j, T2*& base, int& i0) {
+        const int t = tid + k * BD;
+        const int line = t / G::z.r2;
+        j = t - line * G::z.r2;
+        base = S + line * G::pitch + j * (G::z.r1 + G::pad);
+        i0 = (line + line / G::y.r2 * G::y.r2) * N + j;
+        return Z_TASKS % BD == 0 || t < Z_TASKS;
+    };
+    T we[ZT][RZ], wo[ZT][RZ];
+    auto fetch_real = [&](const T* src, T (&e)[ZT][RZ], T (&o)[ZT][RZ]) {
+#pragma unroll
+        for (int k = 0; k < ZT; k++) {
+            int j, i0;
+            T2* base;
+            if (z_task(k, j, base, i0)) {
+#pragma unroll
+                for (int r = 0; r < RZ; r++) {
+                    e[k][r] = src[i0 + r * G::z.r2];
+                    o[k][r] = src[i0 + r * G::z.r2 + SECOND];
+                }
+            }
+        }
+    };
+    auto fetch_w = [&] {
+        if (has_w) fetch_real(it.w + roff, we, wo);
+    };
+    auto load_twiddles = [&] {
+        for (int m = tid; m < N; m += BD) {
+            Wy[m] = twy[m];
+            Wz[m] = twz[m];
+        }
+    };
+    T qe[ZT][RZ], qo[ZT][RZ];
+    // a fetched spectrum -> real values times factor(coef) / M; COMB: (4 x - q) / 3 against the
+    // values already in q. `between`: loads to issue once the spectrum has left its registers.
+    auto inverse = [&](T2 (&v)[YT][RY], T coef, auto comb, auto&& between) {
+#pragma unroll
+        for (int k = 0; k < YT; k++) {
+            int c, j;
+            if (y_task(k, c, j)) pl.template y_scatter<RY>(v[k], pl.column(c), j);
+        }
+        between();
+        __syncthreads();
+        pl.y_merge();
+        __syncthreads();
+        if constexpr (!K::W_RESIDENT) fetch_w();
+        pl.template z_outer<+1>();
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < ZT; k++) {
+            int j, i0;
+            T2* base;
+            if (z_task(k, j, base, i0)) {
+                T2 u[RZ];
+#pragma unroll
+                for (int r = 0; r < RZ; r++) u[r] = base[r];
+#pragma unroll
+                for (int r = 1; r < RZ; r++) u[r] = cmul(u[r], root<+1>(Wz, r * j));
+                RDft<RZ, +1, T, T2>::run(u);
+#pragma unroll
+                for (int r = 0; r < RZ; r++) {
+                    const T xe = u[r].x * factor<T>(we[k][r], has_w, coef) * inv_m;
+                    const T xo = u[r].y * factor<T>(wo[k][r], has_w, coef) * inv_m;
+                    qe[k][r] = decltype(comb)::value ? ((T)4.0 * xe - qe[k][r]) / (T)3.0 : xe;
+                    qo[k][r] = decltype(comb)::value ? ((T)4.0 * xo - qo[k][r]) / (T)3.0 : xo;
+                }
+            }
+        }
+    };
+    // real values times factor(coef) -> spectrum
+    auto forward = [&](T coef, T2* spec) {
+#pragma unroll
+        for (int k = 0; k < ZT; k++) {
+            int j, i0;
+            T2* base;
+            if (z_task(k, j, base, i0)) {
+                T2 u[RZ];
+#pragma unroll
+                for (int r = 0; r < RZ; r++)
+                    u[r] = T2{qe[k][r] * factor<T>(we[k][r], has_w, coef) * (T)0.5,
+                              qo[k][r] * factor<T>(wo[k][r], has_w, coef) * (T)0.5};
+                RDft<RZ, -1, T, T2>::run(u);
+#pragma unroll
+                for (int r = 1; r < RZ; r++) u[r] = cmul(u[r], root<-1>(Wz, r * j));
+#pragma unroll
+                for (int r = 0; r < RZ; r++) base[r] = u[r];
+            }
+        }
+        __syncthreads();
+        pl.template z_outer<-1>();
+        __syncthreads();
+        pl.y_split();
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < YT; k++) {
+            int c, j;
+            if (y_task(k, c, j)) {
+                T2 v[RY];
+                pl.template y_gather<RY>(v, pl.column(c), j);
+#pragma unroll
+                for (int r = 0; r < RY; r++) spec[(j + r * G::y.r1) * G::sp + c] = v[r];
+            }
+        }
+    };
+
+    int n_out = 1;
+    if constexpr (MODE == SLAB_FWD) {
+        fetch_real(it.qin + roff, qe, qo);
+        fetch_w();
+        load_twiddles();
+        __syncthreads();
+        n_out = it.n_out;
+    } else {
+        T2 v[YT][RY];
+        fetch(it.c0 + coff, v);
+        if constexpr (K::W_RESIDENT) fetch_w();
+        load_twiddles();
+        __syncthreads();
+        if constexpr (MODE == SLAB_INV1) {
+            inverse(v, it.post0, std::false_type{}, [] {});
+        } else {
+            inverse(v, it.post0, std::false_type{}, [&] {
+                if constexpr (K::AHEAD) fetch(it.c1 + coff, v);
+            });
+            if constexpr (!K::AHEAD) fetch(it.c1 + coff, v);
+            __syncthreads();   // the plane's values are read
+            inverse(v, it.post1, std::true_type{}, [] {});
+            n_out = 2;
+        }
+#pragma unroll
+        for (int k = 0; k < ZT; k++) {
+            int j, i0;
+            T2* base;
+            if (z_task(k, j, base, i0)) {
+#pragma unroll
+                for (int r = 0; r < RZ; r++) {
+                    const size_t ie = roff + i0 + r * G::z.r2, io = ie + SECOND;
+                    if (it.mask) {
+                        qe[k][r] *= it.mask[ie];
+                        qo[k][r] *= it.mask[io];
+                    }
+                    if (it.qout) {
+                        it.qout[ie] = qe[k][r];
+                        it.qout[io] = qo[k][r];
+                    }
+                }
+            }
+        }
+        if (!it.forward) return;
+    }
+    forward(it.pre0, it.c0 + coff);
+    if (n_out < 2) return;
+    __syncthreads();   // the plane of the first spectrum is read
+    forward(it.pre1, it.c1 + coff);
+}
+
 // ------------------------------------------------------------------ pencil (x) pass
-// One wavefront per y row and tile of one 128-byte line of kz columns.
+// One wavefront per y row and tile of C kz columns.
 __device__ __forceinline__ void two_wave_sync() {
 #ifdef __HIP_DEVICE_COMPILE__
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -610,27 +726,28 @@ __device__ __forceinline__ void two_wave_sync() {
 #endif
 }
 
-template <typename T>
-__global__ void __launch_bounds__(64) pencil_two_kernel(TwoGeom g, XBatch<T> batch,
-                                                        const typename vec2<T>::type* twx, const T* bx, const T* by,
-                                                        const T* bz) {
+template <int C, typename T, typename G>
+__device__ __forceinline__ void pencil_two(const G& g, int jy, int k0, const XItem<T>& it,
+                                           const typename vec2<T>::type* twx, const T* bx, const T* by, const T* bz) {
     using T2 = typename vec2<T>::type;
-    constexpr int C = 128 / (int)sizeof(T2);
     FTS_DYNAMIC_LDS(smem_raw);
     T2* S = reinterpret_cast<T2*>(smem_raw);
-    const int group = g.x.r2 * C + g.xpad;   // slots of one k1
-    T2* Wx = S + g.x.r1 * group;
+    const int group = two_pencil_group(g.xr2, C, sizeof(T2));   // slots of one k1
+    T2* Wx = S + g.xr1 * group;
     const int lane = threadIdx.x;
     for (int m = lane; m < g.x.L; m += 64) Wx[m] = twx[m];
-    const XItem<T>& it = batch.it[blockIdx.y];
-    const int tiles = (g.nzc + C - 1) / C;
-    const int jy = blockIdx.x / tiles;
-    const int k0 = (blockIdx.x - jy * tiles) * C;
     const int cw = min(C, g.nzc - k0);
     const size_t row = (size_t)g.y.L * g.sp;
     T2* c = it.c + (size_t)jy * g.sp + k0;
     const int table = it.table;
-    const int r1 = g.x.r1, r2 = g.x.r2;
+    const auto r1 = g.xr1;
+    const auto r2 = g.xr2;
+    // FP32: the x line of ky = kz = 0 holds the planes' means, the rest of it is small. The value of
+    // the first plane passes by the transforms (its bond factor is 1) and is added to what they
+    // leave of the differences, so the field's mean is not rounded to an FP32 sum of all points
+    // in every convolution (that error, 4e-8 at random, made up most of Q's after 100 steps).
+    const bool mean = sizeof(T) == sizeof(float) && table >= 0 && jy == 0 && k0 == 0;
+    const T first = mean ? c[0].x : (T)0;
     if (table != -2) {
         two_wave_sync();   // twiddles
         for (int t = lane; t < C * r2; t += 64) {
@@ -641,6 +758,10 @@ __global__ void __launch_bounds__(64) pencil_two_kernel(TwoGeom g, XBatch<T> bat
                 T2 v[R];
 #pragma unroll
                 for (int r = 0; r < R; r++) v[r] = c[(size_t)(r * r2 + j) * row + l];
+                if (mean && l == 0) {
+#pragma unroll
+                    for (int r = 0; r < R; r++) v[r].x -= first;
+                }
                 RDft<R, -1, T, T2>::run(v);
 #pragma unroll
                 for (int r = 1; r < R; r++) v[r] = cmul(v[r], root<-1>(Wx, r * j));
@@ -695,41 +816,81 @@ __global__ void __launch_bounds__(64) pencil_two_kernel(TwoGeom g, XBatch<T> bat
 #pragma unroll
             for (int r = 1; r < R; r++) v[r] = cmul(v[r], root<+1>(Wx, r * j));
             RDft<R, +1, T, T2>::run(v);
+            if (mean && l == 0) {
+                // the slab pass scales by 1 / M rounded to T: the difference belongs to the mean too.
+                // The forward and the inverse transform along x scale the differences by nx.
+                const T nx = (T)g.x.L;
+                const T scale = (T)(1.0 - g.inv_m / (double)(T)g.inv_m);
+#pragma unroll
+                for (int r = 0; r < R; r++) v[r].x = first * nx + (v[r].x - first * nx * scale);
+            }
 #pragma unroll
             for (int r = 0; r < R; r++) c[(size_t)(r * r2 + j) * row + l] = v[r];
         });
     }
 }
 
+// a tile of one 128-byte line per wavefront
+template <typename T>
+__global__ void __launch_bounds__(64) pencil_two_kernel(TwoGeom g, XBatch<T> batch,
+                                                        const typename vec2<T>::type* twx, const T* bx, const T* by,
+                                                        const T* bz) {
+    constexpr int C = 128 / (int)sizeof(typename vec2<T>::type);
+    const int tiles = (g.nzc + C - 1) / C;
+    const int jy = blockIdx.x / tiles;
+    pencil_two<C>(TwoView(g), jy, (blockIdx.x - jy * tiles) * C, batch.it[blockIdx.y], twx, bx, by, bz);
+}
+
+// Pencil tiles narrower than a 128-byte line share that line of a spectrum row (rows start
+// on a line) with SH - 1 neighbours. Workgroups go to the 8 XCDs round-robin by linear id,
+// and each XCD has its own L2, so neighbouring tiles would each fetch the line. The grid
+// then pads a row's tiles to a whole number of lines, and xcd_tile orders the tiles so that
+// the SH tiles of one line get ids 8 apart: one XCD, one fetch.
+template <typename T2, int NL>
+constexpr int cube_pencil_share() {
+    return 128 / (NL * (int)sizeof(T2)) > 1 ? 128 / (NL * (int)sizeof(T2)) : 1;
+}
+template <typename T2, int N, int NL>
+constexpr int cube_pencil_tiles() {
+    constexpr int SH = cube_pencil_share<T2, NL>();
+    return ((N / 2 + 1 + NL - 1) / NL + SH - 1) / SH * SH;
+}
+// tile of block b: b = 8 SH g + 8 s + k (k < 8, s < SH) takes tile SH (8 g + k) + s; a
+// bijection when the grid's x extent is a multiple of 8 SH (N x a multiple of SH, N % 8 == 0)
+template <int SH>
+__device__ __forceinline__ int xcd_tile(int b) {
+    if constexpr (SH == 1) {
+        return b;
+    } else {
+        const int g = b / (8 * SH), r = b - g * 8 * SH;
+        return SH * (8 * g + (r & 7)) + (r >> 3);
+    }
+}
+template <typename T, int N, int NL>
+__global__ void __launch_bounds__(64) pencil_cube_kernel(XBatch<T> batch, const typename vec2<T>::type* twx,
+                                                         const T* bx, const T* by, const T* bz) {
+    using T2 = typename vec2<T>::type;
+    constexpr int TILES = cube_pencil_tiles<T2, N, NL>();
+    static_assert(N % 8 == 0, "the XCD tile order needs a grid extent of a multiple of 8 lines' tiles");
+    const int b = xcd_tile<cube_pencil_share<T2, NL>()>(blockIdx.x);
+    const int jy = b / TILES, k0 = (b - jy * TILES) * NL;
+    if (k0 > N / 2) return;   // a pad tile: the whole wavefront leaves
+    pencil_two<NL>(TwoCube<N, sizeof(T2)>{}, jy, k0, batch.it[blockIdx.y], twx, bx, by, bz);
+}
+
 // ------------------------------------------------------------------ whole steps of flat grids
 // A grid of one x-slab (one and two dimensions) holds its whole transform in one workgroup's
 // LDS: the bond factors apply between the forward and the inverse y stage B in registers, and a
 // workgroup runs all consecutive steps of a propagator in one launch.
-template <typename T>
-struct FlatItem {
-    T* q;            // slice n0; slice n0 + s at + s stride
-    T* half;         // continuous: one field of scratch (the full step's result)
-    const T* w;      // as SlabItem::w
-    const T* mask;
-    T full_w, half_w;        // factor coefficients: continuous exp(-w ds/2), exp(-w ds/4); discrete exp(-w ds), unused
-    int steps;
-    int full_table, half_table;
-};
-
-constexpr int FLAT_BATCH = 32;
-template <typename T>
-struct FlatBatch {
-    int n;
-    size_t stride;
-    FlatItem<T> it[FLAT_BATCH];
-};
-
 template <typename T, bool CONTINUOUS>
-__global__ void __launch_bounds__(TWO_BD) flat_steps_kernel(TwoGeom g, FlatBatch<T> batch,
+__global__ void __launch_bounds__(TWO_BD) flat_steps_kernel(TwoGeom geom, FlatBatch<T> batch,
                                                             const typename vec2<T>::type* twy,
                                                             const typename vec2<T>::type* twz, const T* by,
                                                             const T* bz) {
     using T2 = typename vec2<T>::type;
+    using Plane = TwoPlane<T, TwoView>;
+    const TwoView g(geom);
+    const int bd = blockDim.x;
     FTS_DYNAMIC_LDS(smem_raw);
     T2* S = reinterpret_cast<T2*>(smem_raw);
     T2* Wy = S + g.lines * g.pitch;
@@ -737,9 +898,9 @@ __global__ void __launch_bounds__(TWO_BD) flat_steps_kernel(TwoGeom g, FlatBatch
     for (int m = threadIdx.x; m < g.y.L; m += blockDim.x) Wy[m] = twy[m];
     for (int m = threadIdx.x; m < g.z.L; m += blockDim.x) Wz[m] = twz[m];
     const FlatItem<T>& it = batch.it[blockIdx.x];
-    const int second = g.y.r2 * g.z.L;
+    const int second = g.yr2 * g.z.L;
     const T inv_m = (T)g.inv_m;
-    const TwoPlane<T> pl{g, S, Wy, Wz, (int)threadIdx.x, (int)blockDim.x};
+    const Plane pl{g, S, Wy, Wz, (int)threadIdx.x, bd};
     const T* mask = it.mask;
     // convolutions per step: continuous full step, half step, half step; discrete one
     constexpr int NCONV = CONTINUOUS ? 3 : 1;
@@ -797,18 +958,18 @@ __global__ void __launch_bounds__(TWO_BD) flat_steps_kernel(TwoGeom g, FlatBatch
         const int table = CONTINUOUS && next > 0 ? it.half_table : it.full_table;
         const T* ty = by + (size_t)table * g.y.L;
         const T* tz = bz + (size_t)table * g.nzc;
-        const int total = g.nzc * g.y.r1;
+        const int total = g.nzc * g.yr1;
         for (int t = pl.tid; t < total; t += pl.bd) {
             const int j = two_div(t, g.m_nzc), c = t - j * g.nzc;
-            const typename TwoPlane<T>::Col q = pl.column(c);
-            two_radix_call<T>(g.y.r2, [&](auto RC) {
+            const typename Plane::Col q = pl.column(c);
+            two_radix_call<T>(g.yr2, [&](auto RC) {
                 constexpr int R = decltype(RC)::value;
                 T2 v[R];
                 pl.template y_gather<R>(v, q, j);
                 const T b = tz[c];
 #pragma unroll
                 for (int r = 0; r < R; r++) {
-                    const T f = ty[j + r * g.y.r1] * b;
+                    const T f = ty[j + r * g.yr1] * b;
                     v[r] = T2{v[r].x * f, v[r].y * f};
                 }
                 pl.template y_scatter<R>(v, q, j);

@@ -136,64 +136,6 @@ void allow_lds_ct() {
     allow_lds(&xpass_kernel_ct<float, N>);
 }
 
-// Launch-shape candidates of the wave-local kernels (the autotuner's search space)
-constexpr bool slab_bd_ok(int N, int bd) {
-    return (N == 32 && (bd == 128 || bd == 256)) || (N == 48 && (bd == 256 || bd == 384)) ||
-           (N == 64 && (bd == 256 || bd == 320 || bd == 512)) || (N == 96 && (bd == 512 || bd == 1024)) ||
-           (N == 128 && (bd == 512 || bd == 1024));
-}
-constexpr int SLAB_BD_ALL[] = {128, 256, 320, 384, 512, 1024};
-constexpr int PENCIL_NL_ALL[] = {4, 8, 16};
-
-template <typename T, int N, int BD>
-void launch_slab_wl(const Grid& g, int mode, const SlabBatch<T>& b) {
-    using G = WSlab<N, BD>;
-    const dim3 grid(N, b.n), block(BD);
-    const size_t lds = G::lds_elems * sizeof(typename vec2<T>::type);
-    if (mode == SLAB_FWD)
-        hipLaunchKernelGGL((slab_kernel_wl<T, SLAB_FWD, N, BD>), grid, block, lds, g.stream(), b, g.tw<T>(1),
-                           g.tw<T>(2), g.sg.inv_m);
-    else if (mode == SLAB_INV1)
-        hipLaunchKernelGGL((slab_kernel_wl<T, SLAB_INV1, N, BD>), grid, block, lds, g.stream(), b, g.tw<T>(1),
-                           g.tw<T>(2), g.sg.inv_m);
-    else
-        hipLaunchKernelGGL((slab_kernel_wl<T, SLAB_INV2, N, BD>), grid, block, lds, g.stream(), b, g.tw<T>(1),
-                           g.tw<T>(2), g.sg.inv_m);
-}
-
-template <typename T, int N>
-void launch_slab_wl_bd(const Grid& g, int bd, int mode, const SlabBatch<T>& b) {
-    switch (bd) {
-        case 128: if constexpr (slab_bd_ok(N, 128)) return launch_slab_wl<T, N, 128>(g, mode, b); break;
-        case 256: if constexpr (slab_bd_ok(N, 256)) return launch_slab_wl<T, N, 256>(g, mode, b); break;
-        case 320: if constexpr (slab_bd_ok(N, 320)) return launch_slab_wl<T, N, 320>(g, mode, b); break;
-        case 384: if constexpr (slab_bd_ok(N, 384)) return launch_slab_wl<T, N, 384>(g, mode, b); break;
-        case 512: if constexpr (slab_bd_ok(N, 512)) return launch_slab_wl<T, N, 512>(g, mode, b); break;
-        case 1024: if constexpr (slab_bd_ok(N, 1024)) return launch_slab_wl<T, N, 1024>(g, mode, b); break;
-        default: break;
-    }
-    throw Error("no wave-local slab kernel of " + std::to_string(bd) + " threads for N=" + std::to_string(N));
-}
-
-template <typename T, int N, int NL>
-void launch_xpass_wl(const Grid& g, const XBatch<T>& b, const T* bx, const T* by, const T* bz) {
-    using G = WPencil<N, NL>;
-    const dim3 grid(N * wpencil_tiles<typename vec2<T>::type, N, NL>(), b.n), block(G::BD);
-    hipLaunchKernelGGL((xpass_kernel_wl<T, N, NL>), grid, block, G::lds_elems * sizeof(typename vec2<T>::type),
-                       g.stream(), b, g.tw<T>(0), bx, by, bz);
-}
-
-template <typename T, int N>
-void launch_xpass_wl_nl(const Grid& g, int nl, const XBatch<T>& b, const T* bx, const T* by, const T* bz) {
-    switch (nl) {
-        case 4: return launch_xpass_wl<T, N, 4>(g, b, bx, by, bz);
-        case 8: return launch_xpass_wl<T, N, 8>(g, b, bx, by, bz);
-        case 16: return launch_xpass_wl<T, N, 16>(g, b, bx, by, bz);
-        default: break;
-    }
-    throw Error("no wave-local pencil kernel of " + std::to_string(nl) + " columns");
-}
-
 template <typename T, int N, int NL>
 int launch_stress_wl(const Grid& g, const StressBatch<T>& b, const StressGeom& sg, const T* bx, const T* by,
                      const T* bz, double* partials) {
@@ -204,55 +146,21 @@ int launch_stress_wl(const Grid& g, const StressBatch<T>& b, const StressGeom& s
     return N * G::TILES;
 }
 
-template <typename T, int N>
-int launch_stress_wl_nl(const Grid& g, int nl, const StressBatch<T>& b, const StressGeom& sg, const T* bx,
-                        const T* by, const T* bz, double* partials) {
-    switch (nl) {
-        case 4: return launch_stress_wl<T, N, 4>(g, b, sg, bx, by, bz, partials);
-        case 8: return launch_stress_wl<T, N, 8>(g, b, sg, bx, by, bz, partials);
-        case 16: return launch_stress_wl<T, N, 16>(g, b, sg, bx, by, bz, partials);
-        default: break;
-    }
-    throw Error("no wave-local stress kernel of " + std::to_string(nl) + " columns");
-}
-
 template <typename T>
 constexpr int prec_index() {
     return std::is_same<T, float>::value ? 1 : 0;
 }
 
-// LDS limits of every wave-local variant, set before any launch (and so before any
-// graph capture could record the first one)
-template <typename T, int N, int BD>
-void allow_lds_slab_wl() {
-    if constexpr (slab_bd_ok(N, BD)) {
-        allow_lds(&slab_kernel_wl<T, SLAB_FWD, N, BD>);
-        allow_lds(&slab_kernel_wl<T, SLAB_INV1, N, BD>);
-        allow_lds(&slab_kernel_wl<T, SLAB_INV2, N, BD>);
-    }
-}
-
 template <typename T, int N>
-void allow_lds_wl() {
-    allow_lds_slab_wl<T, N, 128>();
-    allow_lds_slab_wl<T, N, 256>();
-    allow_lds_slab_wl<T, N, 320>();
-    allow_lds_slab_wl<T, N, 384>();
-    allow_lds_slab_wl<T, N, 512>();
-    allow_lds_slab_wl<T, N, 1024>();
-    allow_lds(&xpass_kernel_wl<T, N, 4>);
-    allow_lds(&xpass_kernel_wl<T, N, 8>);
-    allow_lds(&xpass_kernel_wl<T, N, 16>);
-    allow_lds(&stress_pencil_wl<T, N, 4>);
-    allow_lds(&stress_pencil_wl<T, N, 8>);
-    allow_lds(&stress_pencil_wl<T, N, 16>);
+void allow_lds_stress() {
+    allow_lds(&stress_pencil_wl<T, N, 128 / (int)sizeof(typename vec2<T>::type)>);
 }
 
 template <int N>
 void allow_lds_n() {
     allow_lds_ct<N>();
-    allow_lds_wl<double, N>();
-    allow_lds_wl<float, N>();
+    allow_lds_stress<double, N>();
+    allow_lds_stress<float, N>();
 }
 
 void set_lds_attributes_ct() {
@@ -263,24 +171,18 @@ void set_lds_attributes_ct() {
     allow_lds_n<64>();
     allow_lds_n<96>();
     allow_lds_n<128>();
+    cube_set_lds_limits<double>();
+    cube_set_lds_limits<float>();
     done = true;
 }
 
 template <typename T, int N>
 void launch_slab_ct(const Grid& g, int mode, const SlabBatch<T>& b) {
     if (g.wave_local) {
-        if constexpr (N > 64) {
-            // at these sizes the wave-local kernel parks the Richardson q1 in the output
-            // slice and starts a second forward transform from qin / qout
-            for (int i = 0; i < b.n; i++) {
-                const SlabItem<T>& it = b.it[i];
-                if ((mode == SLAB_INV2 && !it.qout) || (mode == SLAB_FWD && it.n_out > 1 && !it.qin))
-                    throw Error("slab item without the real slice its second pass reads (N=" + std::to_string(N) + ")");
-            }
-        }
-        const int bd_mode = g.slab_bd_mode[prec_index<T>()][mode];
-        const int bd = bd_mode ? bd_mode : g.slab_bd[prec_index<T>()];
-        launch_slab_wl_bd<T, N>(g, bd ? bd : wslab_default_bd(N), mode, b);
+        const int p = prec_index<T>();
+        int bd = g.slab_bd_mode[p][mode] ? g.slab_bd_mode[p][mode] : g.slab_bd[p];
+        if (!g.schedule_set[p] && N * b.n > SLAB_BATCH_BLOCKS && slab_batch_bd(N, mode)) bd = slab_batch_bd(N, mode);
+        launch_slab_cube<T>(g, N, bd ? bd : slab_default_bd(N), mode, b);
         return;
     }
     using G = SlabShape<N>;
@@ -301,46 +203,13 @@ template <typename T, int N>
 void launch_xpass_ct(const Grid& g, const XBatch<T>& b, const T* bx, const T* by, const T* bz) {
     if (g.wave_local) {
         const int nl = g.pencil_nl[prec_index<T>()];
-        launch_xpass_wl_nl<T, N>(g, nl ? nl : wpencil_default_nl(N, (int)sizeof(typename vec2<T>::type)), b, bx,
-                                 by, bz);
+        launch_pencil_cube<T>(g, N, nl ? nl : pencil_default_nl(N, (int)sizeof(typename vec2<T>::type)), b, bx, by, bz);
         return;
     }
     using G = PencilShape<N>;
     const dim3 grid(N * G::TILES, b.n), block(G::BD);
     hipLaunchKernelGGL((xpass_kernel_ct<T, N>), grid, block, G::lds_elems * sizeof(typename vec2<T>::type), g.stream(),
                        b, g.tw<T>(0), bx, by, bz);
-}
-
-// two-stage kernels: LDS limits, and their launches
-template <typename T>
-void set_lds_attributes_two() {
-    static bool done = false;
-    if (done) return;
-    allow_lds(&slab_two_kernel<T>);
-    allow_lds(&pencil_two_kernel<T>);
-    allow_lds(&flat_steps_kernel<T, true>);
-    allow_lds(&flat_steps_kernel<T, false>);
-    done = true;
-}
-
-template <typename T>
-void launch_slab_two(const Grid& g, int mode, const SlabBatch<T>& b) {
-    // the first half step of a Richardson pair waits in the output slice
-    for (int i = 0; i < b.n; i++)
-        if (mode == SLAB_INV2 && !b.it[i].qout) throw Error("slab item without the real slice its second pass reads");
-    const TwoGeom& t = g.two[prec_index<T>()];
-    hipLaunchKernelGGL((slab_two_kernel<T>), dim3(g.tnx[0], b.n), dim3(two_slab_threads(t)),
-                       two_slab_lds(t, sizeof(typename vec2<T>::type)), g.stream(), t, mode, b, g.tw<T>(1),
-                       g.tw<T>(2));
-}
-
-template <typename T>
-void launch_xpass_two(const Grid& g, const XBatch<T>& b, const T* bx, const T* by, const T* bz) {
-    const TwoGeom& t = g.two[prec_index<T>()];
-    constexpr int e = sizeof(typename vec2<T>::type);
-    const int tiles = ceil_div(t.nzc, two_pencil_columns(e));
-    hipLaunchKernelGGL((pencil_two_kernel<T>), dim3(g.tnx[1] * tiles, b.n), dim3(64), two_pencil_lds(t, e), g.stream(),
-                       t, b, g.tw<T>(0), bx, by, bz);
 }
 
 template <typename T, int MODE, int MAXR, bool BIG>
@@ -495,11 +364,11 @@ void Grid::setup_fft() {
         two_stage[1] = !big && two_geometry(tnx, sizeof(float2), LDS_LIMIT, two[1]);
         if (two_stage[0]) {
             spitch = two[0].sp;
-            set_lds_attributes_two<double>();
+            two_set_lds_limits<double>();
         }
         if (two_stage[1]) {
             spitch32 = two[1].sp;
-            set_lds_attributes_two<float>();
+            two_set_lds_limits<float>();
         }
         Ms = (size_t)tnx[0] * tnx[1] * std::max(spitch, spitch32);
     }
@@ -584,16 +453,14 @@ TuneChoice tune_wave_local(const Grid& g) {
         it.c0 = spec.as<T2>() + 2 * i * Mc;
         it.c1 = spec.as<T2>() + (2 * i + 1) * Mc;
         it.w = w.as<T>();
-        // FP64 discrete steps read exp(-w ds) from a table (coef < 0), FP32 steps evaluate it
-        it.post0 = it.pre0 = std::is_same<T, double>::value ? (T)-1 : (T)0.01;
-        it.post1 = it.pre1 = (T)0.01;
+        it.post0 = it.pre0 = it.post1 = it.pre1 = (T)FACTOR_TABLE;
         it.n_out = 1;
         it.forward = 1;
         xb.it[i].c = spec.as<T2>() + 2 * i * Mc;
         xb.it[i].table = 0;
     }
     const T* bx = tab.as<T>();
-    TuneChoice c{wslab_default_bd(N), wpencil_default_nl(N, (int)sizeof(T2)), "", {0, 0, 0}};
+    TuneChoice c{slab_default_bd(N), pencil_default_nl(N, (int)sizeof(T2)), "", {0, 0, 0}};
     // whole steps (slab pass then pencil pass, as the propagators alternate them)
     std::string note = "us per step of 2 propagators, slab threads/pencil columns";
     float t_def = 0.f, t_best = 1e30f;
@@ -602,8 +469,8 @@ TuneChoice tune_wave_local(const Grid& g) {
         if (!slab_bd_ok(N, bd)) continue;
         for (int nl : PENCIL_NL_ALL) {
             const float t = time_launches(st, [&] {
-                launch_slab_wl_bd<T, N>(g, bd, SLAB_INV1, sb);
-                launch_xpass_wl_nl<T, N>(g, nl, xb, bx, bx + N, bx + 2 * N);
+                launch_slab_cube<T>(g, N, bd, SLAB_INV1, sb);
+                launch_pencil_cube<T>(g, N, nl, xb, bx, bx + N, bx + 2 * N);
             });
             note += us_text(bd, nl, t);
             if (bd == c.bd && nl == c.nl) t_def = t;
@@ -623,7 +490,7 @@ TuneChoice tune_wave_local(const Grid& g) {
     // among the candidates, timed alone (the pencil pass does not depend on it)
     SlabBatch<T> sc = sb;
     for (int i = 0; i < ITEMS; i++) {
-        sc.it[i].post0 = sc.it[i].pre0 = (T)0.01;
+        sc.it[i].post0 = sc.it[i].pre0 = (T)FACTOR_SQUARE;
         sc.it[i].n_out = 2;
     }
     for (int mode : {SLAB_FWD, SLAB_INV2}) {
@@ -632,7 +499,7 @@ TuneChoice tune_wave_local(const Grid& g) {
         int bd_m = c.bd;
         for (int bd : SLAB_BD_ALL) {
             if (!slab_bd_ok(N, bd)) continue;
-            const float t = time_launches(st, [&] { launch_slab_wl_bd<T, N>(g, bd, mode, sc); });
+            const float t = time_launches(st, [&] { launch_slab_cube<T>(g, N, bd, mode, sc); });
             char buf[32];
             std::snprintf(buf, sizeof(buf), " %d:%.2f", bd, 1e3 * t);
             note += buf;
@@ -653,9 +520,9 @@ TuneChoice tune_wave_local(const Grid& g) {
 template <typename T>
 void Grid::tune_fft_schedule() {
     const int p = prec_index<T>();
-    slab_bd[p] = wslab_default_bd(ct_n);
-    for (int m = 0; m < 3; m++) slab_bd_mode[p][m] = 0;
-    pencil_nl[p] = wpencil_default_nl(ct_n, (int)sizeof(typename vec2<T>::type));
+    slab_bd[p] = slab_default_bd(ct_n);
+    for (int m = 0; m < 3; m++) slab_bd_mode[p][m] = slab_default_bd_mode(ct_n, (int)sizeof(typename vec2<T>::type), m);
+    pencil_nl[p] = pencil_default_nl(ct_n, (int)sizeof(typename vec2<T>::type));
     // Tuning picks launch shapes by wall-clock timing, so the choice can differ between
     // processes. At 32^3 and 64^3 every candidate gives bit-identical results; at 48^3,
     // 96^3 and 128^3 they differ by rounding, and a run could then follow another
@@ -686,8 +553,8 @@ void Grid::tune_fft_schedule() {
             }
         } catch (const Error& e) {
             (void)hipGetLastError();
-            c = TuneChoice{wslab_default_bd(ct_n), wpencil_default_nl(ct_n, (int)sizeof(typename vec2<T>::type)),
-                           std::string("defaults (tuning failed: ") + e.what() + ")", {0, 0, 0}};
+            c = TuneChoice{slab_bd[p], pencil_nl[p], std::string("defaults (tuning failed: ") + e.what() + ")", {0, 0, 0}};
+            for (int m = 0; m < 3; m++) c.bd_mode[m] = slab_bd_mode[p][m];
         }
         hit = cache.emplace(key, c).first;
     }
@@ -705,6 +572,7 @@ void Grid::set_fft_schedule(int precision, int threads, int columns) {
     FTS_REQUIRE(columns == 4 || columns == 8 || columns == 16, "pencil columns must be 4, 8 or 16");
     slab_bd[precision] = threads;
     for (int m = 0; m < 3; m++) slab_bd_mode[precision][m] = 0;
+    schedule_set[precision] = true;
     pencil_nl[precision] = columns;
     fft_schedule[precision] = "set by the caller";
 }
@@ -786,7 +654,7 @@ void Grid::launch_slab(int mode, const SlabBatch<T>& b) const {
         case 128: launch_slab_ct<T, 128>(*this, mode, b); break;
         default: {
             if (two_stage[prec_index<T>()]) {
-                launch_slab_two<T>(*this, mode, b);
+                launch_slab_two<T>(mode, b);
                 break;
             }
             const dim3 grid(tnx[0], b.n), block(slab_threads);
@@ -815,7 +683,7 @@ void Grid::launch_xpass(const XBatch<T>& b, const T* bx, const T* by, const T* b
         case 128: launch_xpass_ct<T, 128>(*this, b, bx, by, bz); break;
         default: {
             if (two_stage[prec_index<T>()]) {
-                launch_xpass_two<T>(*this, b, bx, by, bz);
+                launch_xpass_two<T>(b, bx, by, bz);
                 break;
             }
             const dim3 grid(tnx[1] * xg.n_tiles, b.n), block(x_threads);
@@ -833,29 +701,6 @@ void Grid::launch_xpass(const XBatch<T>& b, const T* bx, const T* by, const T* b
 }
 
 template <typename T>
-void Grid::launch_flat(bool continuous, const FlatBatch<T>& b, const T* by, const T* bz) const {
-    require_supported<T>(*this);
-    if (b.n == 0) return;
-    FTS_REQUIRE(flat<T>(), "flat steps need a grid of one x-slab with a two-stage plan");
-    const TwoGeom& t = two[prec_index<T>()];
-    const dim3 grid(b.n), block(two_slab_threads(t));
-    const size_t lds = two_slab_lds(t, sizeof(typename vec2<T>::type));
-    KernelTimer& timer = ctx->timer;
-    hipEvent_t start = timer.begin(stream(), FTS_KERNEL_SLAB);
-    if (continuous)
-        hipLaunchKernelGGL((flat_steps_kernel<T, true>), grid, block, lds, stream(), t, b, tw<T>(1), tw<T>(2), by, bz);
-    else
-        hipLaunchKernelGGL((flat_steps_kernel<T, false>), grid, block, lds, stream(), t, b, tw<T>(1), tw<T>(2), by, bz);
-    FTS_HIP_CHECK(hipGetLastError());
-    if (start) {
-        // each step writes its slice once; the first slice, w and the mask are read once
-        double bytes = 0.0;
-        for (int i = 0; i < b.n; i++) bytes += (double)sizeof(T) * M * (b.it[i].steps + 2 + (b.it[i].mask ? 1 : 0));
-        timer.end(stream(), start, FTS_KERNEL_SLAB, bytes);
-    }
-}
-
-template <typename T>
 int Grid::launch_stress_pencil(const StressBatch<T>& b, const StressGeom& sg, const T* bx, const T* by, const T* bz,
                                double* partials) const {
     require_supported<T>(*this);
@@ -863,14 +708,14 @@ int Grid::launch_stress_pencil(const StressBatch<T>& b, const StressGeom& sg, co
     // tiles of one 128-byte line per spectrum row (rows start on a line): narrower tiles
     // share lines with their neighbours, which run on other XCDs with their own L2, and
     // every line is then fetched twice
-    const int nl = 128 / (int)sizeof(typename vec2<T>::type);
+    constexpr int nl = 128 / (int)sizeof(typename vec2<T>::type);
     int blocks = 0;
     switch (ct_n) {
-        case 32: blocks = launch_stress_wl_nl<T, 32>(*this, nl, b, sg, bx, by, bz, partials); break;
-        case 48: blocks = launch_stress_wl_nl<T, 48>(*this, nl, b, sg, bx, by, bz, partials); break;
-        case 64: blocks = launch_stress_wl_nl<T, 64>(*this, nl, b, sg, bx, by, bz, partials); break;
-        case 96: blocks = launch_stress_wl_nl<T, 96>(*this, nl, b, sg, bx, by, bz, partials); break;
-        case 128: blocks = launch_stress_wl_nl<T, 128>(*this, nl, b, sg, bx, by, bz, partials); break;
+        case 32: blocks = launch_stress_wl<T, 32, nl>(*this, b, sg, bx, by, bz, partials); break;
+        case 48: blocks = launch_stress_wl<T, 48, nl>(*this, b, sg, bx, by, bz, partials); break;
+        case 64: blocks = launch_stress_wl<T, 64, nl>(*this, b, sg, bx, by, bz, partials); break;
+        case 96: blocks = launch_stress_wl<T, 96, nl>(*this, b, sg, bx, by, bz, partials); break;
+        case 128: blocks = launch_stress_wl<T, 128, nl>(*this, b, sg, bx, by, bz, partials); break;
         default: throw Error("the fused stress pencil pass needs an N^3 grid of a specialised size");
     }
     FTS_HIP_CHECK(hipGetLastError());
@@ -1045,8 +890,6 @@ template void Grid::launch_slab<double>(int, const SlabBatch<double>&) const;
 template void Grid::launch_slab<float>(int, const SlabBatch<float>&) const;
 template void Grid::launch_xpass<double>(const XBatch<double>&, const double*, const double*, const double*) const;
 template void Grid::launch_xpass<float>(const XBatch<float>&, const float*, const float*, const float*) const;
-template void Grid::launch_flat<double>(bool, const FlatBatch<double>&, const double*, const double*) const;
-template void Grid::launch_flat<float>(bool, const FlatBatch<float>&, const float*, const float*) const;
 template int Grid::launch_stress_pencil<double>(const StressBatch<double>&, const StressGeom&, const double*,
                                                 const double*, const double*, double*) const;
 template int Grid::launch_stress_pencil<float>(const StressBatch<float>&, const StressGeom&, const float*,

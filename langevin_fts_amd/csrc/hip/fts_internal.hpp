@@ -10,7 +10,7 @@
 #include "fts_common.hpp"
 #include "fts_fft.hpp"
 #include "fts_fft_ct.hpp"
-#include "fts_fft_two.hpp"
+#include "fts_two_plan.hpp"
 #include "fts_fft_wl.hpp"
 
 namespace fts {
@@ -124,6 +124,7 @@ public:
     // replaces slab_bd for that mode, 0: slab_bd
     int slab_bd_mode[2][3] = {{0, 0, 0}, {0, 0, 0}};
     int pencil_nl[2] = {0, 0};
+    bool schedule_set[2] = {false, false};   // set_fft_schedule: every launch in the caller's shape
     std::string fft_schedule[2];
     template <typename T>
     void tune_fft_schedule();
@@ -166,6 +167,10 @@ public:
     }
     template <typename T>
     void launch_flat(bool continuous, const FlatBatch<T>& b, const T* by, const T* bz) const;
+    template <typename T>
+    void launch_slab_two(int mode, const SlabBatch<T>& b) const;
+    template <typename T>
+    void launch_xpass_two(const XBatch<T>& b, const T* bx, const T* by, const T* bz) const;
     // The stress of b.n terms from the slab pass's output spectra, with their x transforms
     // fused into the reduction (wave-local grids only): 3 partial sums per workgroup into
     // partials, term-major; returns the workgroups per term.
@@ -192,6 +197,18 @@ public:
     template <typename T>
     void fft_backward_noalloc(const typename vec2<T>::type* in, T* out, int batch);
 };
+
+// LDS limits of the two-stage kernels of a precision; before any launch of them
+template <typename T>
+void two_set_lds_limits();
+template <typename T>
+void cube_set_lds_limits();
+
+// the slab and pencil passes of an n^3 grid in a launch shape of fts_two_plan.hpp
+template <typename T>
+void launch_slab_cube(const Grid& g, int n, int bd, int mode, const SlabBatch<T>& b);
+template <typename T>
+void launch_pencil_cube(const Grid& g, int n, int nl, const XBatch<T>& b, const T* bx, const T* by, const T* bz);
 
 // Looks up the device address of the no-allocation workspace for `device` (which must
 // be current) once per device; called when a context is created.

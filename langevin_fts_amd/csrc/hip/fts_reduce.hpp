@@ -161,7 +161,7 @@ struct InitItem {
     const T* src[INIT_MAX_SRC];
     T coef[INIT_MAX_SRC];
     const double* qinit;
-    const T* w;       // factor exp(-w*wcoef) after the op (nullptr: none)
+    const T* w;       // factor(wcoef) after the op (nullptr: none)
     T wcoef;
     const T* mask;
 };
@@ -188,7 +188,7 @@ __global__ void init_kernel(InitBatch<T> b, int M) {
             v = it.accumulate ? it.dst[i] : (T)1;
             for (int s = 0; s < it.n_src; s++) v *= it.src[s][i];
         }
-        if (it.w) v *= it.wcoef < (T)0 ? it.w[i] : fexp<T>(-it.w[i] * it.wcoef);
+        v *= factor<T>(it.w ? it.w[i] : (T)1, it.w != nullptr, it.wcoef);
         if (it.mask) v *= it.mask[i];
         it.dst[i] = v;
     }
@@ -199,10 +199,11 @@ __global__ void convert_kernel(const double* in, T* out, int M) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < M; i += gridDim.x * blockDim.x) out[i] = (T)in[i];
 }
 
-// out = exp(-w coef), the factor of every discrete step (w fixed during a call)
+// out = exp(-w coef), the factor of every step (w fixed during a call)
 template <typename T>
-__global__ void exp_table_kernel(const T* w, T coef, T* out, int n) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[i] = fexp<T>(-w[i] * coef);
+__global__ void exp_table_kernel(const T* w, double coef, T* out, int n) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        out[i] = (T)exp(-(double)w[i] * coef);
 }
 
 // FP64 fields (one per blockIdx.y) into consecutive fields of the solver's precision

@@ -35,7 +35,8 @@ public:
     void results_changed() override { Q_valid_ = false; }
     std::vector<double> launch_signature() const override {
         const GraphKey k = graph_key(nullptr, nullptr);
-        return {k.volume, (double)k.bd, (double)k.nl, (double)k.bd_fwd, (double)k.bd_inv2, (double)tables_version_};
+        return {k.volume, (double)k.bd, (double)k.nl, (double)k.bd_fwd, (double)k.bd_inv2, (double)k.set,
+                (double)tables_version_};
     }
     void compute_propagators(const double* const* w, const double* const* q_init, bool on_device) override;
     void compute_concentrations() override;
@@ -89,11 +90,16 @@ private:
     }
     T* slice_ptr(int p, int n, int half) const { return half ? h(p, n) : q(p, n); }
     const T* w(int m) const { return wT_ + (size_t)m * M_; }
-    // discrete FP64 chains: exp(-w ds) of monomer m, made once per compute_propagators (the FP32
-    // kernels compute their single-precision exponential on the fly: a table measures the same there)
-    bool table() const { return model_ == FTS_DISCRETE && std::is_same<T, double>::value; }
-    const T* ew(int m) const { return table() ? ew_.as<T>() + (size_t)m * M_ : w(m); }
-    T ew_coef() const { return table() ? (T)-1 : (T)ds_; }   // negative: the array is the factor
+    // the steps' exponential of monomer m, made once per compute_propagators from FP64 exponentials:
+    // exp(-w ds) of discrete chains, exp(-w ds/4) of continuous ones, whose exp(-w ds/2) is its square
+    // (a Richardson step evaluated five exponentials per point, 10% of a 64^3 FP64 evaluation; in
+    // FP32 the time is the same, and the rounded FP64 value has none of the hardware exponential's bias)
+    bool table() const { return !real_; }
+    double table_arg() const { return model_ == FTS_DISCRETE ? ds_ : ds_ / 4; }
+    const T* ew(int m) const { return ew_.as<T>() + (size_t)m * M_; }
+    T ew_full() const { return (T)FACTOR_TABLE; }        // discrete: exp(-w ds)
+    T ew_half() const { return (T)FACTOR_SQUARE; }       // continuous: exp(-w ds/2)
+    T ew_quarter() const { return (T)FACTOR_TABLE; }     // continuous: exp(-w ds/4)
     T2* slot(int s) const { return ws_.as<T2>() + (size_t)s * Ms_; }
     const T* mask() const { return g_->mask_h.empty() ? nullptr : g_->mask<T>(); }
     int full(int m) const { return 2 * m; }
@@ -117,10 +123,10 @@ private:
     struct GraphKey {
         std::vector<const void*> ptrs;
         double volume = 0.0;
-        int bd = 0, nl = 0, bd_fwd = 0, bd_inv2 = 0;
+        int bd = 0, nl = 0, bd_fwd = 0, bd_inv2 = 0, set = 0;
         bool operator==(const GraphKey& o) const {
             return ptrs == o.ptrs && volume == o.volume && bd == o.bd && nl == o.nl && bd_fwd == o.bd_fwd &&
-                   bd_inv2 == o.bd_inv2;
+                   bd_inv2 == o.bd_inv2 && set == o.set;
         }
     };
     GraphKey graph_key(const double* const* w, const double* const* q_init) const;
@@ -512,7 +518,6 @@ void Solver<T>::launch_real(const RealBatch& b) {
 
 template <typename T>
 void Solver<T>::build_slice(const std::vector<std::array<int, 3>>& jobs) {
-    const T ds = (T)ds_;
     // ---- initial slices of propagators starting in this slice
     // rounds of at most INIT_MAX_SRC dependencies; later rounds accumulate
     std::vector<std::vector<InitItem<T>>> rounds;
@@ -565,7 +570,7 @@ void Solver<T>::build_slice(const std::vector<std::array<int, 3>>& jobs) {
                 it.op = pr.kind == FTS_LEAF ? INIT_ONE : INIT_QINIT;
                 if (pr.kind == FTS_LEAF_QINIT) it.qinit = qinit_.as<double>() + (size_t)pr.qinit * M_;
                 it.w = ew(m);
-                it.wcoef = ew_coef();
+                it.wcoef = ew_full();
                 it.mask = mask();
                 add_init(0, it);
             } else {
@@ -606,7 +611,7 @@ void Solver<T>::build_slice(const std::vector<std::array<int, 3>>& jobs) {
             SlabItem<T> b{};
             b.c0 = slot(f.slot);
             b.w = ew(props_[f.p].monomer);
-            b.post0 = ew_coef();
+            b.post0 = ew_full();
             b.mask = mask();
             b.qout = q(f.p, 1);
             inv.push_back(b);
@@ -640,10 +645,10 @@ void Solver<T>::build_slice(const std::vector<std::array<int, 3>>& jobs) {
             FlatItem<T> it{};
             it.q = q(r.p, r.n0);
             it.half = reinterpret_cast<T*>(slot(2 * r.slot));
-            it.w = model_ == FTS_CONTINUOUS ? w(m) : ew(m);
+            it.w = ew(m);
             it.mask = mask();
-            it.full_w = model_ == FTS_CONTINUOUS ? ds / 2 : ew_coef();
-            it.half_w = ds / 4;
+            it.full_w = model_ == FTS_CONTINUOUS ? ew_half() : ew_full();
+            it.half_w = ew_quarter();
             it.steps = r.cnt;
             it.full_table = full(m);
             it.half_table = half(m);
@@ -683,9 +688,9 @@ void Solver<T>::build_slice(const std::vector<std::array<int, 3>>& jobs) {
                     a.qin = q(r.p, n);
                     a.c0 = c0;
                     a.c1 = c1;
-                    a.w = w(m);
-                    a.pre0 = ds / 2;
-                    a.pre1 = ds / 4;
+                    a.w = ew(m);
+                    a.pre0 = ew_half();
+                    a.pre1 = ew_quarter();
                     a.n_out = 2;
                     fw.push_back(a);
                 }
@@ -693,22 +698,22 @@ void Solver<T>::build_slice(const std::vector<std::array<int, 3>>& jobs) {
                 x1.push_back({c1, half(m)});
                 SlabItem<T> b{};
                 b.c0 = c1;
-                b.w = w(m);
-                b.post0 = ds / 2;
+                b.w = ew(m);
+                b.post0 = ew_half();
                 b.forward = 1;
                 inv1.push_back(b);
                 x2.push_back({c1, half(m)});
                 SlabItem<T> c{};
                 c.c0 = c0;
                 c.c1 = c1;
-                c.w = w(m);
-                c.post0 = ds / 2;
-                c.post1 = ds / 4;
+                c.w = ew(m);
+                c.post0 = ew_half();
+                c.post1 = ew_quarter();
                 c.mask = mask();
                 c.qout = q(r.p, n + 1);
                 c.forward = last ? 0 : 1;
-                c.pre0 = ds / 2;
-                c.pre1 = ds / 4;
+                c.pre0 = ew_half();
+                c.pre1 = ew_quarter();
                 inv2.push_back(c);
             } else {
                 T2* c0 = slot(r.slot);
@@ -723,7 +728,7 @@ void Solver<T>::build_slice(const std::vector<std::array<int, 3>>& jobs) {
                 SlabItem<T> b{};
                 b.c0 = c0;
                 b.w = ew(m);
-                b.post0 = ew_coef();
+                b.post0 = ew_full();
                 b.mask = mask();
                 b.qout = q(r.p, n + 1);
                 b.forward = last ? 0 : 1;
@@ -869,6 +874,7 @@ typename Solver<T>::GraphKey Solver<T>::graph_key(const double* const* w, const 
     k.bd_fwd = g_->slab_bd_mode[p][SLAB_FWD];
     k.bd_inv2 = g_->slab_bd_mode[p][SLAB_INV2];
     k.nl = g_->pencil_nl[p];
+    k.set = g_->schedule_set[p] ? 1 : 0;
     return k;
 }
 
@@ -954,7 +960,7 @@ void Solver<T>::issue_propagators(const double* const* wf, const double* const* 
     if (!std::is_same<T, double>::value) FTS_HIP_CHECK(hipGetLastError());
     if (table()) {
         hipLaunchKernelGGL((exp_table_kernel<T>), dim3(std::min(1024, ceil_div(n_mon_ * M_, 256))), dim3(256), 0,
-                           g_->stream(), wT_, (T)ds_, ew_.as<T>(), n_mon_ * M_);
+                           g_->stream(), wT_, table_arg(), ew_.as<T>(), n_mon_ * M_);
         FTS_HIP_CHECK(hipGetLastError());
     }
     for (int i = 0; i < n_qinit_; i++) {

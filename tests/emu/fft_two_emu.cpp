@@ -161,7 +161,7 @@ struct Emu {
         table(bz, n[2], g.nzc);
         std::printf("y %d x %d, z %d x %d, x %d x %d, threads %d, pitch %d, lds %zu + %zu\n", g.y.r1, g.y.r2, g.z.r1,
                     g.z.r2, g.x.r1, g.x.r2, fts::two_slab_threads(g), g.pitch, fts::two_slab_lds(g, sizeof(T2)),
-                    fts::two_pencil_lds(g, sizeof(T2)));
+                    fts::two_pencil_lds(g, fts::two_pencil_columns(sizeof(T2)), sizeof(T2)));
     }
     void slab(int mode, const fts::SlabItem<T>& it) {
         fts::SlabBatch<T> b{};
@@ -175,7 +175,7 @@ struct Emu {
         b.n = 1;
         b.it[0] = fts::XItem<T>{c, table};
         const int C = fts::two_pencil_columns(sizeof(T2));
-        run_grid(dim3{(unsigned)(n[1] * ((g.nzc + C - 1) / C)), 1, 1}, 64, fts::two_pencil_lds(g, sizeof(T2)),
+        run_grid(dim3{(unsigned)(n[1] * ((g.nzc + C - 1) / C)), 1, 1}, 64, fts::two_pencil_lds(g, fts::two_pencil_columns(sizeof(T2)), sizeof(T2)),
                  [&] { fts::pencil_two_kernel<T>(g, b, tw[0].data(), bx.data(), by.data(), bz.data()); });
     }
     std::vector<T2> spectrum() const { return std::vector<T2>(Ms, T2{(T)NAN, (T)NAN}); }
@@ -236,7 +236,10 @@ int run(const char* op, const int* n, const char* in_path, const char* out_path)
     } else {
         // input: q, w, mask
         std::vector<T> w(in.begin() + M, in.begin() + 2 * M), mask(in.begin() + 2 * M, in.begin() + 3 * M);
-        const T ds = (T)0.25;
+        // factors are read from a table: exp(-w ds/4) or, of discrete steps, exp(-w ds)
+        const double ds = 0.25;
+        for (T& x : w) x = (T)std::exp(-(double)x * (is("flatd") ? ds : ds / 4));
+        const T half_w = (T)fts::FACTOR_SQUARE, quarter_w = (T)fts::FACTOR_TABLE, full_w = (T)fts::FACTOR_TABLE;
         out.assign(2 * M, (T)NAN);
         if (is("step")) {
             std::vector<T> q(in.begin(), in.begin() + M);
@@ -246,8 +249,8 @@ int run(const char* op, const int* n, const char* in_path, const char* out_path)
             a.c0 = c0.data();
             a.c1 = c1.data();
             a.w = w.data();
-            a.pre0 = ds / 2;
-            a.pre1 = ds / 4;
+            a.pre0 = half_w;
+            a.pre1 = quarter_w;
             a.n_out = 2;
             e.slab(fts::SLAB_FWD, a);
             for (int s = 0; s < 2; s++) {
@@ -256,7 +259,7 @@ int run(const char* op, const int* n, const char* in_path, const char* out_path)
                 fts::SlabItem<T> b{};
                 b.c0 = c1.data();
                 b.w = w.data();
-                b.post0 = ds / 2;
+                b.post0 = half_w;
                 b.forward = 1;
                 e.slab(fts::SLAB_INV1, b);
                 e.pencil(c1.data(), 1);
@@ -264,8 +267,8 @@ int run(const char* op, const int* n, const char* in_path, const char* out_path)
                 c.c0 = c0.data();
                 c.c1 = c1.data();
                 c.w = w.data();
-                c.post0 = c.pre0 = ds / 2;
-                c.post1 = c.pre1 = ds / 4;
+                c.post0 = c.pre0 = half_w;
+                c.post1 = c.pre1 = quarter_w;
                 c.mask = mask.data();
                 c.qout = out.data() + s * M;
                 c.forward = s == 0;
@@ -286,8 +289,8 @@ int run(const char* op, const int* n, const char* in_path, const char* out_path)
             it.full_table = 0;
             it.half_table = 1;
             const bool cont = is("flat");
-            it.full_w = cont ? ds / 2 : ds;
-            it.half_w = ds / 4;
+            it.full_w = cont ? half_w : full_w;
+            it.half_w = quarter_w;
             run_grid(dim3{1, 1, 1}, fts::two_slab_threads(e.g), fts::two_slab_lds(e.g, sizeof(T2)), [&] {
                 if (cont)
                     fts::flat_steps_kernel<T, true>(e.g, b, e.tw[1].data(), e.tw[2].data(), e.by.data(), e.bz.data());

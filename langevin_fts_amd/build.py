@@ -30,6 +30,12 @@ HIP_FLAGS = [
 ] + os.environ.get("FTS_HIP_DEFINES", "").split()   # tuning defines, e.g. -DFTS_STREAM_STORES=1
 
 
+# The general-size kernels carry a branch per radix: hoisted out of their loops, the FP64 constants
+# and row offsets of all branches fill the scalar registers (337 of them spilled in the slab kernel, 41
+# with the machine-level hoisting off).
+FILE_FLAGS = {"fts_two.hip": ["-mllvm", "-disable-machine-licm"]}
+
+
 def _newer(target, deps):
     if not os.path.exists(target):
         return True
@@ -55,7 +61,7 @@ def build_hip(force=False, jobs=4):
         obj = os.path.join(BUILD, os.path.basename(src) + ".o")
         objs.append(obj)
         if force or _newer(obj, [src] + headers):
-            todo.append([HIPCC] + HIP_FLAGS + ["-c", "-o", obj, src])
+            todo.append([HIPCC] + HIP_FLAGS + FILE_FLAGS.get(os.path.basename(src), []) + ["-c", "-o", obj, src])
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         list(ex.map(_run, todo))
     lib = os.path.join(PKG, "libfts_hip.so")

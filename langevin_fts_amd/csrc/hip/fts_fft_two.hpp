@@ -33,7 +33,7 @@ namespace fts {
 
 // ------------------------------------------------------------------ register transforms
 // RDft<R, DIR>::run: R-point transform in registers, natural order in and out, DIR -1 forward.
-// 2, 3, 4, 5 and 8 are fts_fft.hpp's butterflies; R = A B with coprime A, B by the prime-factor
+// 2, 3, 4 and 5 are fts_fft.hpp's butterflies; R = A B with coprime A, B by the prime-factor
 // algorithm (no twiddles); 9 and 16 as 3 x 3 and 4 x 4; 7, 11 and 13 from the symmetric sums
 // v_j +- v_(R - j).
 template <int R>
@@ -74,6 +74,21 @@ __host__ __device__ constexpr double root_sin(int R, int m) {
     return R == 9 ? s9[m] : s16[m];
 }
 
+// Products are written as fused operations: the compiler's own choice of which product of a sum
+// to fuse can differ between instances of one kernel, and every launch shape of a grid gives the
+// same results.
+__device__ __forceinline__ double two_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float two_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+template <typename T2>
+__device__ __forceinline__ T2 tmul(T2 a, T2 w) {
+    return T2{two_fma(a.x, w.x, -(a.y * w.y)), two_fma(a.x, w.y, a.y * w.x)};
+}
+// a times the conjugate of w
+template <typename T2>
+__device__ __forceinline__ T2 tmul_conj(T2 a, T2 w) {
+    return T2{two_fma(a.x, w.x, a.y * w.y), two_fma(a.y, w.x, -(a.x * w.y))};
+}
+
 template <int R, int DIR, typename T, typename T2>
 struct RDft;
 
@@ -95,7 +110,27 @@ struct RDft<4, DIR, T, T2> : RDftBase<4, DIR, T, T2> {};
 template <int DIR, typename T, typename T2>
 struct RDft<5, DIR, T, T2> : RDftBase<5, DIR, T, T2> {};
 template <int DIR, typename T, typename T2>
-struct RDft<8, DIR, T, T2> : RDftBase<8, DIR, T, T2> {};
+struct RDft<8, DIR, T, T2> {
+    static __device__ __forceinline__ void run(T2 (&v)[8]) {
+        const T h = (T)0.70710678118654752440;
+        T2 e[4] = {v[0], v[2], v[4], v[6]};
+        T2 o[4] = {v[1], v[3], v[5], v[7]};
+        RDft<4, DIR, T, T2>::run(e);
+        RDft<4, DIR, T, T2>::run(o);
+        // o[1] and o[3] times W8 = (1 + DIR i) h and W8^3 = (-1 + DIR i) h, h in the final sums
+        const T2 a = T2{o[1].x - DIR * o[1].y, o[1].y + DIR * o[1].x};
+        const T2 b = T2{-o[3].x - DIR * o[3].y, DIR * o[3].x - o[3].y};
+        const T2 c = mul_is<DIR>(o[2]);
+        v[0] = cadd(e[0], o[0]);
+        v[4] = csub(e[0], o[0]);
+        v[1] = T2{two_fma(a.x, h, e[1].x), two_fma(a.y, h, e[1].y)};
+        v[5] = T2{two_fma(a.x, -h, e[1].x), two_fma(a.y, -h, e[1].y)};
+        v[2] = cadd(e[2], c);
+        v[6] = csub(e[2], c);
+        v[3] = T2{two_fma(b.x, h, e[3].x), two_fma(b.y, h, e[3].y)};
+        v[7] = T2{two_fma(b.x, -h, e[3].x), two_fma(b.y, -h, e[3].y)};
+    }
+};
 
 // coprime A, B: input index (B a + A b) mod R, output k with k mod A = ka and k mod B = kb
 template <int A, int B, int DIR, typename T, typename T2>
@@ -151,7 +186,7 @@ struct RDftSquare {
             for (int a = 1; a < A; a++)
                 if (b > 0) {
                     if (R == 16 && a * b == 4) t[b][a] = mul_is<DIR>(t[b][a]);
-                    else t[b][a] = cmul(t[b][a], T2{(T)root_cos(R, a * b), (T)(DIR * root_sin(R, a * b))});
+                    else t[b][a] = tmul(t[b][a], T2{(T)root_cos(R, a * b), (T)(DIR * root_sin(R, a * b))});
                 }
         }
 #pragma unroll
@@ -244,6 +279,20 @@ __device__ __forceinline__ void two_radix_call(int r, F&& f) {
     }
 }
 
+// v, opaque to the compiler where it is a value of the grid: the products r v of every radix's
+// branch stay in the branch (they cost one scalar multiplication each there). Hoisted out of the
+// loops they fill and spill the scalar registers: 390 spills in the FP64 slab kernel.
+__device__ __forceinline__ int two_opaque(const TwoView&, int v) {
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("" : "+s"(v));
+#endif
+    return v;
+}
+template <int N, int E>
+__device__ __forceinline__ constexpr int two_opaque(const TwoCube<N, E>&, int v) {
+    return v;
+}
+
 // ------------------------------------------------------------------ the plane of a slab
 template <typename T, typename G>
 struct TwoPlane {
@@ -257,6 +306,8 @@ struct TwoPlane {
     struct Col {
         int e, o;
         bool self;    // c = nz - c (mod nz): one value, o is a spare slot
+        // of row k1's values (a choice of values: one between the members would put them in memory)
+        __device__ __forceinline__ int slot(int k1) const { return e + (k1 & 1) * (o - e); }
     };
     __device__ __forceinline__ int zslot(int k) const { return g.pad ? k + two_div(k, g.m_zr1) : k; }
     __device__ __forceinline__ Col column(int c) const {
@@ -270,12 +321,20 @@ struct TwoPlane {
     template <int R>
     __device__ __forceinline__ void y_scatter(T2 (&v)[R], const Col& q, int j) const {
         RDft<R, +1, T, T2>::run(v);
-        T2* base = S + (j >> 1) * g.yr2 * g.pitch + ((j & 1) ? q.o : q.e);
+        const int pitch = two_opaque(g, g.pitch);
+        T2* base = S + (j >> 1) * g.yr2 * pitch + q.slot(j);
 #pragma unroll
-        for (int r = 0; r < R; r++) base[r * g.pitch] = v[r];
+        for (int r = 0; r < R; r++) base[r * pitch] = v[r];
     }
-    // stage A of y, inverse, with the merge of the row pairs
-    __device__ __forceinline__ void y_merge() const {
+    // the LDS table's root for output r of butterfly j
+    struct Table {
+        const T2* W;
+        __device__ __forceinline__ T2 operator()(int r, int j) const { return W[r * j]; }
+    };
+    // stage A of y, inverse, with the merge of the row pairs; w(r, j): the forward root W^(r j)
+    __device__ __forceinline__ void y_merge() const { y_merge(Table{Wy}); }
+    template <typename W>
+    __device__ __forceinline__ void y_merge(const W& w) const {
         const int total = g.nzc * g.yr2;
         for (int t = tid; t < total; t += bd) {
             const int j = two_div(t, g.m_nzc), c = t - j * g.nzc;
@@ -283,18 +342,20 @@ struct TwoPlane {
             two_radix_call<T>(g.yr1, [&](auto RC) {
                 constexpr int R = decltype(RC)::value;
                 T2 v[R];
+                const int pair = two_opaque(g, g.yr2 * g.pitch);   // from line (a, j) to (a + 1, j)
+                T2* const even = S + j * g.pitch + q.e;
+                T2* const odd = S + j * g.pitch + q.o;
 #pragma unroll
-                for (int r = 0; r < R; r++) v[r] = S[((r >> 1) * g.yr2 + j) * g.pitch + ((r & 1) ? q.o : q.e)];
+                for (int r = 0; r < R; r++) v[r] = ((r & 1) ? odd : even)[(r >> 1) * pair];
 #pragma unroll
-                for (int r = 1; r < R; r++) v[r] = cmul(v[r], root<+1>(Wy, r * j));
+                for (int r = 1; r < R; r++) v[r] = tmul_conj(v[r], w(r, j));
                 RDft<R, +1, T, T2>::run(v);
 #pragma unroll
                 for (int a = 0; a < (R + 1) / 2; a++) {
                     T2 A = v[2 * a], B = 2 * a + 1 < R ? v[(2 * a + 1) % R] : T2{(T)0, (T)0};
                     if (q.self) A.y = B.y = (T)0;
-                    T2* base = S + (a * g.yr2 + j) * g.pitch;
-                    base[q.e] = T2{A.x - B.y, A.y + B.x};
-                    if (!q.self) base[q.o] = T2{A.x + B.y, B.x - A.y};
+                    even[a * pair] = T2{A.x - B.y, A.y + B.x};
+                    if (!q.self) odd[a * pair] = T2{A.x + B.y, B.x - A.y};
                 }
             });
         }
@@ -302,13 +363,14 @@ struct TwoPlane {
     // stage B of z: inverse (k natural -> (k1, n2)) or forward ((k1, n2) -> k natural)
     template <int DIR>
     __device__ __forceinline__ void z_outer() const {
-        const int total = g.lines * g.zr1, step = g.zr1 + g.pad;
+        const int total = g.lines * g.zr1;
         for (int t = tid; t < total; t += bd) {
             const int line = two_div(t, g.m_zr1), j = t - line * g.zr1;
             T2* base = S + line * g.pitch + j;
             two_radix_call<T>(g.zr2, [&](auto RC) {
                 constexpr int R = decltype(RC)::value;
                 T2 v[R];
+                const int step = two_opaque(g, g.zr1 + g.pad);
 #pragma unroll
                 for (int r = 0; r < R; r++) v[r] = base[r * step];
                 RDft<R, DIR, T, T2>::run(v);
@@ -338,15 +400,16 @@ struct TwoPlane {
 #pragma unroll
                     for (int r = 0; r < R; r++) v[r] = base[r];
 #pragma unroll
-                    for (int r = 1; r < R; r++) v[r] = cmul(v[r], root<+1>(Wz, r * j));
+                    for (int r = 1; r < R; r++) v[r] = tmul_conj(v[r], Wz[r * j]);
                     RDft<R, +1, T, T2>::run(v);
                 }
+                const int run = two_opaque(g, g.zr2);
 #pragma unroll
-                for (int r = 0; r < R; r++) op(i0 + r * g.zr2, two, v[r]);
+                for (int r = 0; r < R; r++) op(i0 + r * run, two, v[r]);
                 if (forward) {
                     RDft<R, -1, T, T2>::run(v);
 #pragma unroll
-                    for (int r = 1; r < R; r++) v[r] = cmul(v[r], root<-1>(Wz, r * j));
+                    for (int r = 1; r < R; r++) v[r] = tmul(v[r], Wz[r * j]);
 #pragma unroll
                     for (int r = 0; r < R; r++) base[r] = v[r];
                 }
@@ -355,7 +418,9 @@ struct TwoPlane {
     }
     // stage A of y, forward, with the split of the packed lines (twice the rows' spectra: the
     // caller halves the real values)
-    __device__ __forceinline__ void y_split() const {
+    __device__ __forceinline__ void y_split() const { y_split(Table{Wy}); }
+    template <typename W>
+    __device__ __forceinline__ void y_split(const W& w) const {
         const int total = g.nzc * g.yr2;
         for (int t = tid; t < total; t += bd) {
             const int j = two_div(t, g.m_nzc), c = t - j * g.nzc;
@@ -363,28 +428,31 @@ struct TwoPlane {
             two_radix_call<T>(g.yr1, [&](auto RC) {
                 constexpr int R = decltype(RC)::value;
                 T2 v[R];
+                const int pair = two_opaque(g, g.yr2 * g.pitch);
+                T2* const even = S + j * g.pitch + q.e;
+                T2* const odd = S + j * g.pitch + q.o;
 #pragma unroll
                 for (int a = 0; a < (R + 1) / 2; a++) {
-                    const T2* base = S + (a * g.yr2 + j) * g.pitch;
-                    const T2 A = base[q.e];
-                    const T2 B = q.self ? A : base[q.o];
+                    const T2 A = even[a * pair];
+                    const T2 B = q.self ? A : odd[a * pair];
                     v[2 * a] = T2{A.x + B.x, A.y - B.y};
                     if (2 * a + 1 < R) v[(2 * a + 1) % R] = T2{A.y + B.y, B.x - A.x};
                 }
                 RDft<R, -1, T, T2>::run(v);
 #pragma unroll
-                for (int r = 1; r < R; r++) v[r] = cmul(v[r], root<-1>(Wy, r * j));
+                for (int r = 1; r < R; r++) v[r] = tmul(v[r], w(r, j));
 #pragma unroll
-                for (int r = 0; r < R; r++) S[((r >> 1) * g.yr2 + j) * g.pitch + ((r & 1) ? q.o : q.e)] = v[r];
+                for (int r = 0; r < R; r++) ((r & 1) ? odd : even)[(r >> 1) * pair] = v[r];
             });
         }
     }
     // stage B of y, forward: v[r] becomes row j + r1 r of the column
     template <int R>
     __device__ __forceinline__ void y_gather(T2 (&v)[R], const Col& q, int j) const {
-        const T2* base = S + (j >> 1) * g.yr2 * g.pitch + ((j & 1) ? q.o : q.e);
+        const int pitch = two_opaque(g, g.pitch);
+        const T2* base = S + (j >> 1) * g.yr2 * pitch + q.slot(j);
 #pragma unroll
-        for (int r = 0; r < R; r++) v[r] = base[r * g.pitch];
+        for (int r = 0; r < R; r++) v[r] = base[r * pitch];
         RDft<R, -1, T, T2>::run(v);
     }
 };
@@ -437,9 +505,10 @@ __device__ __forceinline__ void slab_two(const G& g, int mode, int bd, const Sla
                 two_radix_call<T>(g.yr2, [&](auto RC) {
                     constexpr int R = decltype(RC)::value;
                     T2 v[R];
-                    const T2* src = spec + (size_t)j * g.sp + c;
+                    const T2* src = spec + j * g.sp + c;
+                    const int rows = two_opaque(g, g.yr1 * g.sp);
 #pragma unroll
-                    for (int r = 0; r < R; r++) v[r] = src[r * g.yr1 * g.sp];
+                    for (int r = 0; r < R; r++) v[r] = src[r * rows];
                     pl.template y_scatter<R>(v, q, j);
                 });
             }
@@ -483,9 +552,10 @@ __device__ __forceinline__ void slab_two(const G& g, int mode, int bd, const Sla
                 constexpr int R = decltype(RC)::value;
                 T2 v[R];
                 pl.template y_gather<R>(v, q, j);
-                T2* dst = spec + (size_t)j * g.sp + c;
+                T2* dst = spec + j * g.sp + c;
+                const int rows = two_opaque(g, g.yr1 * g.sp);
 #pragma unroll
-                for (int r = 0; r < R; r++) dst[r * g.yr1 * g.sp] = v[r];
+                for (int r = 0; r < R; r++) dst[r * rows] = v[r];
             });
         }
     }
@@ -502,7 +572,7 @@ __global__ void __launch_bounds__(TWO_BD) slab_two_kernel(TwoGeom g, int mode, S
 // the inverse to the last forward transform, and every global load is issued a phase or more before
 // its use: the first spectrum and w before the first barrier, the second spectrum of a
 // Richardson step when the first has left its registers.
-template <typename T, int N, int BD>
+template <typename T, int MODE, int N, int BD>
 struct CubeSlab {
     using T2 = typename vec2<T>::type;
     using G = TwoCube<N, sizeof(T2)>;
@@ -516,13 +586,22 @@ struct CubeSlab {
     static constexpr bool W_RESIDENT = WORDS * (2 * 2 * ZT * RZ + 2 * 16) <= VGPRS - 40;
     // the second spectrum is loaded ahead when that many registers are left
     static constexpr bool AHEAD = WORDS * (2 * 2 * ZT * RZ + 2 * YT * RY + 2 * 16) <= VGPRS - 40;
+    // Where every stage has at most one butterfly per thread, the roots a thread needs can stay in
+    // registers, read from the tables in HBM before the first barrier, instead of 4 (r1 - 1) LDS
+    // reads per transform pair. The shapes of few workgroups do: 64^3 with 320 threads 9.3 -> 8.9 and
+    // 15.8 -> 15.2 us (half step, Richardson step of two propagators in FP64), 32^3 5.1 -> 4.8. In the
+    // shapes of large batches the registers cost workgroups per CU (64^3 with 512 threads, 16
+    // propagators: 27 -> 37 us; the Richardson step of 32 propagators at 32^3: 14.6 -> 18.1 us).
+    static constexpr bool ROOTS =
+        (sizeof(T) == 8 && N == 64 && BD == 320) || (N == 32 && BD == 256 && MODE != SLAB_INV2);
+    static_assert(!ROOTS || (ZT == 1 && G::nzc * G::y.r2 <= BD), "one butterfly per thread");
 };
 
 template <typename T, int MODE, int N, int BD>
 __global__ void __launch_bounds__(BD) slab_cube_kernel(SlabBatch<T> batch, const typename vec2<T>::type* twy,
                                                        const typename vec2<T>::type* twz) {
     using T2 = typename vec2<T>::type;
-    using K = CubeSlab<T, N, BD>;
+    using K = CubeSlab<T, MODE, N, BD>;
     using G = typename K::G;
     using Plane = TwoPlane<T, G>;
     constexpr int YT = K::YT, ZT = K::ZT, RY = K::RY, RZ = K::RZ;
@@ -584,12 +663,24 @@ __global__ void __launch_bounds__(BD) slab_cube_kernel(SlabBatch<T> batch, const
     auto fetch_w = [&] {
         if (has_w) fetch_real(it.w + roff, we, wo);
     };
+    constexpr int NR = K::ROOTS ? 1 : 0;
+    T2 ry[NR * G::y.r1 + 1], rz[NR * G::z.r1 + 1];
     auto load_twiddles = [&] {
-        for (int m = tid; m < N; m += BD) {
-            Wy[m] = twy[m];
-            Wz[m] = twz[m];
+        if constexpr (K::ROOTS) {
+            const int jy = min(tid / G::nzc, G::y.r2 - 1), jz = tid % G::z.r2;
+#pragma unroll
+            for (int r = 1; r < G::y.r1; r++) ry[r] = twy[r * jy];
+#pragma unroll
+            for (int r = 1; r < G::z.r1; r++) rz[r] = twz[r * jz];
+        } else {
+            for (int m = tid; m < N; m += BD) {
+                Wy[m] = twy[m];
+                Wz[m] = twz[m];
+            }
         }
     };
+    auto y_root = [&](int r, int j) { return K::ROOTS ? ry[NR * r] : Wy[r * j]; };
+    auto z_root = [&](int r, int j) { return K::ROOTS ? rz[NR * r] : Wz[r * j]; };
     T qe[ZT][RZ], qo[ZT][RZ];
     // a fetched spectrum -> real values times factor(coef) / M; COMB: (4 x - q) / 3 against the
     // values already in q. `between`: loads to issue once the spectrum has left its registers.
@@ -601,7 +692,7 @@ __global__ void __launch_bounds__(BD) slab_cube_kernel(SlabBatch<T> batch, const
         }
         between();
         __syncthreads();
-        pl.y_merge();
+        pl.y_merge(y_root);
         __syncthreads();
         if constexpr (!K::W_RESIDENT) fetch_w();
         pl.template z_outer<+1>();
@@ -615,7 +706,7 @@ __global__ void __launch_bounds__(BD) slab_cube_kernel(SlabBatch<T> batch, const
 #pragma unroll
                 for (int r = 0; r < RZ; r++) u[r] = base[r];
 #pragma unroll
-                for (int r = 1; r < RZ; r++) u[r] = cmul(u[r], root<+1>(Wz, r * j));
+                for (int r = 1; r < RZ; r++) u[r] = tmul_conj(u[r], z_root(r, j));
                 RDft<RZ, +1, T, T2>::run(u);
 #pragma unroll
                 for (int r = 0; r < RZ; r++) {
@@ -641,7 +732,7 @@ __global__ void __launch_bounds__(BD) slab_cube_kernel(SlabBatch<T> batch, const
                               qo[k][r] * factor<T>(wo[k][r], has_w, coef) * (T)0.5};
                 RDft<RZ, -1, T, T2>::run(u);
 #pragma unroll
-                for (int r = 1; r < RZ; r++) u[r] = cmul(u[r], root<-1>(Wz, r * j));
+                for (int r = 1; r < RZ; r++) u[r] = tmul(u[r], z_root(r, j));
 #pragma unroll
                 for (int r = 0; r < RZ; r++) base[r] = u[r];
             }
@@ -649,7 +740,7 @@ __global__ void __launch_bounds__(BD) slab_cube_kernel(SlabBatch<T> batch, const
         __syncthreads();
         pl.template z_outer<-1>();
         __syncthreads();
-        pl.y_split();
+        pl.y_split(y_root);
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < YT; k++) {
@@ -737,7 +828,7 @@ __device__ __forceinline__ void pencil_two(const G& g, int jy, int k0, const XIt
     const int lane = threadIdx.x;
     for (int m = lane; m < g.x.L; m += 64) Wx[m] = twx[m];
     const int cw = min(C, g.nzc - k0);
-    const size_t row = (size_t)g.y.L * g.sp;
+    const int row = g.y.L * g.sp;
     T2* c = it.c + (size_t)jy * g.sp + k0;
     const int table = it.table;
     const auto r1 = g.xr1;
@@ -756,17 +847,19 @@ __device__ __forceinline__ void pencil_two(const G& g, int jy, int k0, const XIt
             two_radix_call<T>(r1, [&](auto RC) {
                 constexpr int R = decltype(RC)::value;
                 T2 v[R];
+                const T2* src = c + (size_t)(j * row + l);
+                const int next = two_opaque(g, r2 * row);
 #pragma unroll
-                for (int r = 0; r < R; r++) v[r] = c[(size_t)(r * r2 + j) * row + l];
+                for (int r = 0; r < R; r++) v[r] = src[r * next];
                 if (mean && l == 0) {
 #pragma unroll
                     for (int r = 0; r < R; r++) v[r].x -= first;
                 }
                 RDft<R, -1, T, T2>::run(v);
 #pragma unroll
-                for (int r = 1; r < R; r++) v[r] = cmul(v[r], root<-1>(Wx, r * j));
+                for (int r = 1; r < R; r++) v[r] = tmul(v[r], Wx[r * j]);
 #pragma unroll
-                for (int r = 0; r < R; r++) S[r * group + j * C + l] = v[r];
+                for (int r = 0; r < R; r++) S[r * two_opaque(g, group) + j * C + l] = v[r];
             });
         }
         two_wave_sync();
@@ -784,19 +877,20 @@ __device__ __forceinline__ void pencil_two(const G& g, int jy, int k0, const XIt
                 RDft<R, -1, T, T2>::run(v);
                 if (table == -1) {
 #pragma unroll
-                    for (int r = 0; r < R; r++) c[(size_t)(j + r * r1) * row + l] = v[r];
+                    for (int r = 0; r < R; r++) c[(j + r * r1) * row + l] = v[r];
                     return;
                 }
                 const T* tx = bx + (size_t)table * g.x.L + j;
                 const T bl = by[(size_t)table * g.y.L + jy] * bz[(size_t)table * g.nzc + k0 + l];
+                const int next = two_opaque(g, r1);
 #pragma unroll
                 for (int r = 0; r < R; r++) {
-                    const T b = tx[r * r1] * bl;
+                    const T b = tx[r * next] * bl;
                     v[r] = T2{v[r].x * b, v[r].y * b};
                 }
             } else {
 #pragma unroll
-                for (int r = 0; r < R; r++) v[r] = c[(size_t)(j + r * r1) * row + l];
+                for (int r = 0; r < R; r++) v[r] = c[(j + r * r1) * row + l];
             }
             RDft<R, +1, T, T2>::run(v);
 #pragma unroll
@@ -812,9 +906,9 @@ __device__ __forceinline__ void pencil_two(const G& g, int jy, int k0, const XIt
             constexpr int R = decltype(RC)::value;
             T2 v[R];
 #pragma unroll
-            for (int r = 0; r < R; r++) v[r] = S[r * group + j * C + l];
+            for (int r = 0; r < R; r++) v[r] = S[r * two_opaque(g, group) + j * C + l];
 #pragma unroll
-            for (int r = 1; r < R; r++) v[r] = cmul(v[r], root<+1>(Wx, r * j));
+            for (int r = 1; r < R; r++) v[r] = tmul_conj(v[r], Wx[r * j]);
             RDft<R, +1, T, T2>::run(v);
             if (mean && l == 0) {
                 // the slab pass scales by 1 / M rounded to T: the difference belongs to the mean too.
@@ -825,7 +919,7 @@ __device__ __forceinline__ void pencil_two(const G& g, int jy, int k0, const XIt
                 for (int r = 0; r < R; r++) v[r].x = first * nx + (v[r].x - first * nx * scale);
             }
 #pragma unroll
-            for (int r = 0; r < R; r++) c[(size_t)(r * r2 + j) * row + l] = v[r];
+            for (int r = 0; r < R; r++) c[r * two_opaque(g, r2 * row) + j * row + l] = v[r];
         });
     }
 }
@@ -967,9 +1061,10 @@ __global__ void __launch_bounds__(TWO_BD) flat_steps_kernel(TwoGeom geom, FlatBa
                 T2 v[R];
                 pl.template y_gather<R>(v, q, j);
                 const T b = tz[c];
+                const int rows = two_opaque(g, g.yr1);
 #pragma unroll
                 for (int r = 0; r < R; r++) {
-                    const T f = ty[j + r * g.yr1] * b;
+                    const T f = ty[j + r * rows] * b;
                     v[r] = T2{v[r].x * f, v[r].y * f};
                 }
                 pl.template y_scatter<R>(v, q, j);
@@ -980,6 +1075,126 @@ __global__ void __launch_bounds__(TWO_BD) flat_steps_kernel(TwoGeom geom, FlatBa
         __syncthreads();
         pl.template z_outer<+1>();
         __syncthreads();
+    }
+}
+
+// ------------------------------------------------------------------ whole steps in one dimension
+// A line of up to LINE_POINTS points takes its convolutions directly: the bond factors' inverse
+// transform is a row of n coefficients, and a thread group sums a point's n products, every
+// value in LDS or registers. Two barriers per Richardson step (a buffer is written again only two
+// barriers after its readers), where two butterflies each way and
+// the row pairing (with an empty partner) take eighteen: a step of 128 points took 23 us by
+// flat_steps_kernel, bound by those phases' latency, and takes 0.9 us. Sums are FP64 in either
+// precision.
+template <typename T, bool CONTINUOUS, int P, int CH>
+__global__ void __launch_bounds__(1024) line_steps_kernel(int n, FlatBatch<T> batch, const T* bz) {
+    FTS_DYNAMIC_LDS(smem_raw);
+    double* full = reinterpret_cast<double*>(smem_raw);   // coefficients of the full and the half bond
+    double* half = full + n;
+    double* xa = half + n;                                // inputs of the three convolutions, two buffers each
+    double* xb = xa + 2 * n;
+    double* xc = xb + 2 * n;
+    const FlatItem<T>& it = batch.it[blockIdx.x];
+    const int nzc = n / 2 + 1;
+    // P neighbouring lanes share point i; lane p takes the inputs j = p (mod P)
+    const int i = threadIdx.x / P, p = threadIdx.x % P;
+    const bool on = i < n;
+    for (int m = threadIdx.x; m < n; m += blockDim.x) {
+        // cos(2 pi m / n) by its symmetries, so that a period's values cancel
+        const int h = min(m, n - m);
+        xa[m] = 4 * h <= n ? cospi(2.0 * h / n) : -cospi((double)(n - 2 * h) / n);
+        if (m < nzc) {
+            xb[m] = (double)bz[(size_t)it.full_table * nzc + m];
+            if (CONTINUOUS) xc[m] = (double)bz[(size_t)it.half_table * nzc + m];
+        }
+    }
+    __syncthreads();
+    for (int m = threadIdx.x; m < (CONTINUOUS ? 2 : 1) * n; m += blockDim.x) {
+        const int d = m < n ? m : m - n;
+        const double* b = m < n ? xb : xc;
+        // compensated: the coefficients' errors act the same way in every step
+        double sum = b[0], lost = 0.0;
+        int a = 0;   // k d mod n
+        for (int k = 1; k < nzc; k++) {
+            a += d;
+            if (a >= n) a -= n;
+            const double y = (2 * k == n ? 1.0 : 2.0) * (b[k] * xa[a]) - lost;
+            const double next = sum + y;
+            lost = (next - sum) - y;
+            sum = next;
+        }
+        full[m] = sum / n;
+    }
+    __syncthreads();
+    if (threadIdx.x < (CONTINUOUS ? 2 : 1)) {
+        // the coefficients add up to b[0]: what rounding left of that would scale the field's mean
+        // in every step
+        double* c = threadIdx.x == 0 ? full : half;
+        double left = threadIdx.x == 0 ? xb[0] : xc[0], lost = 0.0;
+        for (int k = 0; k < n; k++) {
+            const double y = -c[k] - lost, next = left + y;
+            lost = (next - left) - y;
+            left = next;
+        }
+        c[0] += left;
+    }
+    __syncthreads();
+    T* q = it.q;
+    const double f = on ? (double)it.w[i] : 0.0;
+    // discrete: exp(-w ds); continuous: exp(-w ds/4) and its square, rounded as the slab passes' are
+    const double e4 = f, e2 = CONTINUOUS ? (double)((T)f * (T)f) : 0.0;
+    const double mask = on && it.mask ? (double)it.mask[i] : 1.0;
+    double x = on ? (double)q[i] : 0.0;
+    // this lane's coefficients c[(i - j) mod n] of j = p + P t, and the places of v[j]: in registers
+    // for all steps (CH of them, those beyond the line zero), or read from the LDS (CH 0)
+    double cf[CH + 1], ch[CH + 1];
+#pragma unroll
+    for (int t = 0; t < CH; t++) {
+        const int j = p + P * t, d = i - j;
+        const bool valid = on && j < n;
+        cf[t] = valid ? full[d < 0 ? d + n : d] : 0.0;
+        ch[t] = CONTINUOUS && valid ? half[d < 0 ? d + n : d] : 0.0;
+    }
+    // sum over j of c[(i - j) mod n] v[j], in every lane of the group
+    auto conv = [&](const double (&reg)[CH + 1], const double* c, const double* v) {
+        double s = 0.0;
+        if constexpr (CH > 0) {
+#pragma unroll
+            for (int t = 0; t < CH; t++) s += reg[t] * v[min(p + P * t, n - 1)];
+        } else if (on) {
+            int d = i - p;
+            if (d < 0) d += n;
+            for (int j = p; j < n; j += P) {
+                s += c[d] * v[j];
+                d -= P;
+                if (d < 0) d += n;
+            }
+        }
+#pragma unroll
+        for (int m = 1; m < P; m <<= 1) s += __shfl_xor(s, m, 64);
+        return s;
+    };
+    for (int s = 0; s < it.steps; s++) {
+        double* a = xa + (s & 1) * n;
+        double* b = xb + (s & 1) * n;
+        double* c = xc + (s & 1) * n;
+        if (on && p == 0) {
+            a[i] = CONTINUOUS ? e2 * x : x;
+            if (CONTINUOUS) b[i] = e4 * x;
+        }
+        __syncthreads();
+        if constexpr (CONTINUOUS) {
+            const double q1 = e2 * conv(cf, full, a);
+            const double t = e2 * conv(ch, half, b);
+            if (on && p == 0) c[i] = t;
+            __syncthreads();
+            x = (4.0 * (e4 * conv(ch, half, c)) - q1) / 3.0 * mask;
+        } else {
+            x = e4 * conv(cf, full, a) * mask;
+        }
+        x = (double)(T)x;   // the stored slice is what the next step starts from
+        q += batch.stride;
+        if (on && p == 0) q[i] = (T)x;
     }
 }
 

@@ -276,7 +276,9 @@ Solver<T>::Solver(Grid* grid, const fts_plan* pl, const int* bc, bool reduce_mem
     }
     if (table()) ew_.allocate(sizeof(T) * n_mon_ * (size_t)M_);
     if (n_qinit_) qinit_.allocate(sizeof(double) * n_qinit_ * (size_t)M_);
-    n_ws_ = std::max<int>(2 * (int)jmax, 16);
+    // at least 8 stress terms per chunk, and 32 where their spectra stay below 64 MB: a chunk of
+    // a small grid is bound by its launches (128 points: 13 chunks took 270 us of an evaluation)
+    n_ws_ = std::max<int>(2 * (int)jmax, sizeof(T2) * 2 * MAX_BATCH * Ms_ <= ((size_t)64 << 20) ? 2 * MAX_BATCH : 16);
     ws_.allocate(sizeof(T2) * (size_t)n_ws_ * Ms_);
     phib_.allocate(sizeof(double) * blocks_.size() * (size_t)M_);
     if (!svf_.empty()) phis_.allocate(sizeof(double) * svf_.size() * (size_t)M_);
@@ -936,31 +938,16 @@ void Solver<T>::issue_propagators(const double* const* wf, const double* const* 
     const int cb = std::min(1024, ceil_div(M_, 256));
     for (int m = 0; m < n_mon_; m++) {
         FTS_REQUIRE(wf[m] != nullptr, "missing field for a monomer type");
-        if (std::is_same<T, double>::value) {
+        if (!on_device)
             FTS_HIP_CHECK(hipMemcpyAsync(w64_.as<double>() + (size_t)m * M_, wf[m], sizeof(double) * M_, kind,
                                          g_->stream()));
-        } else if (on_device) {
-            continue;   // converted below, straight from the caller's device fields
-        } else {
-            FTS_HIP_CHECK(hipMemcpyAsync(w64_.as<double>() + (size_t)m * M_, wf[m], sizeof(double) * M_, kind,
-                                         g_->stream()));
-            hipLaunchKernelGGL((convert_kernel<T>), dim3(cb), dim3(256), 0, g_->stream(),
-                               w64_.as<double>() + (size_t)m * M_, wT_ + (size_t)m * M_, M_);
-        }
     }
-    if (!std::is_same<T, double>::value && on_device) {
-        for (int m0 = 0; m0 < n_mon_; m0 += MAX_BATCH) {
-            ConvertBatch cv{};
-            cv.n = std::min(MAX_BATCH, n_mon_ - m0);
-            for (int k = 0; k < cv.n; k++) cv.src[k] = wf[m0 + k];
-            hipLaunchKernelGGL((convert_batch_kernel<T>), dim3(cb, cv.n), dim3(256), 0, g_->stream(), cv,
-                               wT_ + (size_t)m0 * M_, M_);
-        }
-    }
-    if (!std::is_same<T, double>::value) FTS_HIP_CHECK(hipGetLastError());
-    if (table()) {
-        hipLaunchKernelGGL((exp_table_kernel<T>), dim3(std::min(1024, ceil_div(n_mon_ * M_, 256))), dim3(256), 0,
-                           g_->stream(), wT_, table_arg(), ew_.as<T>(), n_mon_ * M_);
+    for (int m0 = 0; m0 < n_mon_; m0 += MAX_BATCH) {
+        FieldBatch fb{};
+        fb.n = std::min(MAX_BATCH, n_mon_ - m0);
+        for (int k = 0; k < fb.n; k++) fb.src[k] = on_device ? wf[m0 + k] : w64_.as<double>() + (size_t)(m0 + k) * M_;
+        hipLaunchKernelGGL((fields_kernel<T>), dim3(cb, fb.n), dim3(256), 0, g_->stream(), fb, table_arg(),
+                           wT_ + (size_t)m0 * M_, table() ? ew_.as<T>() + (size_t)m0 * M_ : nullptr, M_);
         FTS_HIP_CHECK(hipGetLastError());
     }
     for (int i = 0; i < n_qinit_; i++) {

@@ -57,7 +57,16 @@ void Grid::launch_flat(bool continuous, const FlatBatch<T>& b, const T* by, cons
     const size_t lds = two_slab_lds(t, sizeof(typename vec2<T>::type));
     KernelTimer& timer = ctx->timer;
     hipEvent_t start = timer.begin(stream(), FTS_KERNEL_SLAB);
-    if (continuous)
+    const int n = tnx[2], P = line_lanes(n);
+    if (tnx[1] == 1 && n <= LINE_POINTS) {
+        const dim3 threads(ceil_div(n * P, 64) * 64);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, threads, line_lds(n), stream(), n, b, bz);
+        };
+        if (n <= 64) go(continuous ? line_steps_kernel<T, true, 8, 8> : line_steps_kernel<T, false, 8, 8>);
+        else if (n <= 128) go(continuous ? line_steps_kernel<T, true, 8, 16> : line_steps_kernel<T, false, 8, 16>);
+        else go(continuous ? line_steps_kernel<T, true, 4, 0> : line_steps_kernel<T, false, 4, 0>);
+    } else if (continuous)
         hipLaunchKernelGGL((flat_steps_kernel<T, true>), grid, block, lds, stream(), t, b, tw<T>(1), tw<T>(2), by, bz);
     else
         hipLaunchKernelGGL((flat_steps_kernel<T, false>), grid, block, lds, stream(), t, b, tw<T>(1), tw<T>(2), by, bz);

@@ -204,4 +204,10 @@ struct FlatBatch {
     FlatItem<T> it[FLAT_BATCH];
 };
 
+// Points of a line that takes its convolutions directly (n products per point), and the lanes that
+// share a point: at most 1024 threads
+constexpr int LINE_POINTS = 256;
+constexpr int line_lanes(int n) { return n <= 128 ? 8 : 4; }
+constexpr size_t line_lds(int n) { return sizeof(double) * 8 * (size_t)n; }
+
 }  // namespace fts

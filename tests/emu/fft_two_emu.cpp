@@ -15,6 +15,7 @@
 //          forward, INV2 with forward), twice; input: q, w, mask; output: both slices
 //    flat: the same two steps by flat_steps_kernel (nx = 1)
 //    flatd: two discrete steps by flat_steps_kernel (nx = 1)
+//    line, lined: the same by line_steps_kernel with one lane per point (nx = ny = 1)
 // Bond factors along each axis: exp(-0.3 (k / L)^2) full, exp(-0.15 (k / L)^2) half, k folded.
 #include <hip/hip_runtime.h>
 
@@ -31,6 +32,8 @@
 namespace fts {
 unsigned char* smem_raw_ptr;
 }
+inline double cospi(double x) { return std::cos(M_PI * x); }
+inline double __shfl_xor(double v, int, int) { return v; }   // groups of one lane only
 #define FTS_DYNAMIC_LDS(name) unsigned char* name = smem_raw_ptr
 #include "fts_fft_two.hpp"
 
@@ -238,7 +241,7 @@ int run(const char* op, const int* n, const char* in_path, const char* out_path)
         std::vector<T> w(in.begin() + M, in.begin() + 2 * M), mask(in.begin() + 2 * M, in.begin() + 3 * M);
         // factors are read from a table: exp(-w ds/4) or, of discrete steps, exp(-w ds)
         const double ds = 0.25;
-        for (T& x : w) x = (T)std::exp(-(double)x * (is("flatd") ? ds : ds / 4));
+        for (T& x : w) x = (T)std::exp(-(double)x * (is("flatd") || is("lined") ? ds : ds / 4));
         const T half_w = (T)fts::FACTOR_SQUARE, quarter_w = (T)fts::FACTOR_TABLE, full_w = (T)fts::FACTOR_TABLE;
         out.assign(2 * M, (T)NAN);
         if (is("step")) {
@@ -288,9 +291,15 @@ int run(const char* op, const int* n, const char* in_path, const char* out_path)
             it.steps = 2;
             it.full_table = 0;
             it.half_table = 1;
-            const bool cont = is("flat");
+            const bool cont = is("flat") || is("line");
             it.full_w = cont ? half_w : full_w;
             it.half_w = quarter_w;
+            if (is("line") || is("lined")) {
+                run_grid(dim3{1, 1, 1}, (n[2] + 63) / 64 * 64, fts::line_lds(n[2]), [&] {
+                    if (cont) fts::line_steps_kernel<T, true, 1, 0>(n[2], b, e.bz.data());
+                    else fts::line_steps_kernel<T, false, 1, 128>(n[2], b, e.bz.data());
+                });
+            } else
             run_grid(dim3{1, 1, 1}, fts::two_slab_threads(e.g), fts::two_slab_lds(e.g, sizeof(T2)), [&] {
                 if (cont)
                     fts::flat_steps_kernel<T, true>(e.g, b, e.tw[1].data(), e.tw[2].data(), e.by.data(), e.bz.data());

@@ -2,7 +2,7 @@
 tests/emu/fft_two_emu.cpp and run as emulated workgroups with AddressSanitizer on the LDS block
 and on every global buffer (NaN in what was never written): forward and inverse transforms
 against numpy, a convolution with the bond factors, and two masked propagator steps of each kind
-by the slab and pencil passes and by the one-launch kernel of flat grids, against numpy in FP64.
+by the slab and pencil passes and by the one-launch kernels of flat grids, against numpy in FP64.
 The grids take every radix 1..16 on the axes, odd and even lengths (rows without a partner, no
 Nyquist column), more butterflies than threads, and the plans' limits. CPU only.
 
@@ -79,7 +79,7 @@ def check(exe, n, esize, ops, tmp):
         else:
             out, x = [], q
             for _ in range(2):
-                if op == "flatd":
+                if op in ("flatd", "lined"):
                     x = np.exp(-w * ds) * conv(n, x, 1.0) * mask
                 else:
                     e2, e4 = np.exp(-w * ds / 2), np.exp(-w * ds / 4)
@@ -93,6 +93,10 @@ def check(exe, n, esize, ops, tmp):
         assert e < tol, (n, esize, op, e)
 
 
+def flat_ops(n):
+    return (["flat", "flatd"] if n[0] == 1 else []) + (["line", "lined"] if n[0] == n[1] == 1 else [])
+
+
 # (x, y, z): every radix as r1 and as r2 of a y and of a z plan, odd and even lengths
 GRIDS = [(2, 8, 8), (3, 6, 10), (4, 12, 9), (5, 15, 16), (7, 14, 26), (11, 22, 33), (13, 21, 35), (2, 45, 20),
          (6, 7, 13), (1, 60, 104), (1, 1, 128), (1, 1, 30), (2, 30, 27), (9, 10, 1), (16, 3, 4), (2, 49, 25),
@@ -101,11 +105,11 @@ GRIDS = [(2, 8, 8), (3, 6, 10), (4, 12, 9), (5, 15, 16), (7, 14, 26), (11, 22, 3
 
 @pytest.mark.parametrize("n", GRIDS)
 def test_two_stage_fp64(exe, n, tmp_path):
-    ops = ["fft", "ifft", "conv", "step"] + (["flat", "flatd"] if n[0] == 1 else [])
+    ops = ["fft", "ifft", "conv", "step"] + flat_ops(n)
     check(exe, n, 8, ops, str(tmp_path))
 
 
 @pytest.mark.parametrize("n", [(2, 8, 8), (3, 6, 10), (5, 15, 16), (1, 20, 48), (1, 1, 128)])
 def test_two_stage_fp32(exe, n, tmp_path):
-    ops = ["fft", "ifft", "conv", "step"] + (["flat", "flatd"] if n[0] == 1 else [])
+    ops = ["fft", "ifft", "conv", "step"] + flat_ops(n)
     check(exe, n, 4, ops, str(tmp_path))

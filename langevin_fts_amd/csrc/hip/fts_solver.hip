@@ -91,11 +91,11 @@ private:
     T* slice_ptr(int p, int n, int half) const { return half ? h(p, n) : q(p, n); }
     const T* w(int m) const { return wT_ + (size_t)m * M_; }
     // the steps' exponential of monomer m, made once per compute_propagators from FP64 exponentials:
-    // exp(-w ds) of discrete chains, exp(-w ds/4) of continuous ones, whose exp(-w ds/2) is its square
+    // exp(-w ds) of discrete chains, exp(-w ds/4) of continuous ones, whose exp(-w ds/2) is its square,
+    // exp(-w ds/2) of real-space steps
     // (a Richardson step evaluated five exponentials per point, 10% of a 64^3 FP64 evaluation; in
     // FP32 the time is the same, and the rounded FP64 value has none of the hardware exponential's bias)
-    bool table() const { return !real_; }
-    double table_arg() const { return model_ == FTS_DISCRETE ? ds_ : ds_ / 4; }
+    double table_arg() const { return model_ == FTS_DISCRETE ? ds_ : real_ ? ds_ / 2 : ds_ / 4; }
     const T* ew(int m) const { return ew_.as<T>() + (size_t)m * M_; }
     T ew_full() const { return (T)FACTOR_TABLE; }        // discrete: exp(-w ds)
     T ew_half() const { return (T)FACTOR_SQUARE; }       // continuous: exp(-w ds/2)
@@ -274,7 +274,7 @@ Solver<T>::Solver(Grid* grid, const fts_plan* pl, const int* bc, bool reduce_mem
         w32_.allocate(sizeof(float) * n_mon_ * (size_t)M_);
         wT_ = reinterpret_cast<T*>(w32_.as<float>());
     }
-    if (table()) ew_.allocate(sizeof(T) * n_mon_ * (size_t)M_);
+    ew_.allocate(sizeof(T) * n_mon_ * (size_t)M_);
     if (n_qinit_) qinit_.allocate(sizeof(double) * n_qinit_ * (size_t)M_);
     // at least 8 stress terms per chunk, and 32 where their spectra stay below 64 MB: a chunk of
     // a small grid is bound by its launches (128 points: 13 chunks took 270 us of an evaluation)
@@ -301,7 +301,6 @@ Solver<T>::Solver(Grid* grid, const fts_plan* pl, const int* bc, bool reduce_mem
             off += RT_ROWS * g_->nx[a] + 2;
         }
         rg_.tab_stride = off;
-        rg_.half_ds = 0.5 * ds_;
         rtab_.allocate(sizeof(double) * (size_t)off * n_mon_);
         build_real_tables();
     } else {
@@ -476,6 +475,11 @@ void Solver<T>::launch_real(const RealBatch& b) {
             while (t.P * RT_LMAX < A.n) t.P <<= 1;
             t.Lc = ceil_div(A.n, t.P);
             t.R = RT_THREADS / t.P;
+            while ((1 << t.log2R) < t.R) t.log2R++;
+            // 64 KiB hold the tile and the four coefficient rows at an odd pitch for every even
+            // length but the longest, 64 RT_LMAX
+            t.pitch = A.n < 64 * RT_LMAX ? A.n | 1 : A.n;
+            t.m_n = two_recip(A.n);
             const bool inner = A.iax == 2;
             int blocks;
             if (inner) {
@@ -485,7 +489,7 @@ void Solver<T>::launch_real(const RealBatch& b) {
                 blocks = rg_.tn[A.iax == 0 ? 1 : 0] * t.ktiles;
             }
             const dim3 grid(blocks, b.n);
-            const size_t lds = sizeof(double) * (size_t)(t.R + 4) * A.n;
+            const size_t lds = sizeof(double) * ((size_t)t.R * t.pitch + 4 * (size_t)A.n);
 #define FTS_REAL_TILED(F, L, I)                                                                                \
     hipLaunchKernelGGL((real_tiled_kernel<F, L, I>), grid, dim3(RT_THREADS), lds, g_->stream(), b, rg_, tab, a, t)
             if (inner) {
@@ -675,7 +679,7 @@ void Solver<T>::build_slice(const std::vector<std::array<int, 3>>& jobs) {
                     it.qe = reinterpret_cast<double*>(slot(2 * r.slot));
                     it.acc = reinterpret_cast<double*>(slot(2 * r.slot + 1));
                     it.qout = q(r.p, n + 1);
-                    it.w = w(m);
+                    it.w = ew(m);
                     it.mask = mask();
                     it.monomer = m;
                     it.need_pre = t == start;
@@ -947,7 +951,7 @@ void Solver<T>::issue_propagators(const double* const* wf, const double* const* 
         fb.n = std::min(MAX_BATCH, n_mon_ - m0);
         for (int k = 0; k < fb.n; k++) fb.src[k] = on_device ? wf[m0 + k] : w64_.as<double>() + (size_t)(m0 + k) * M_;
         hipLaunchKernelGGL((fields_kernel<T>), dim3(cb, fb.n), dim3(256), 0, g_->stream(), fb, table_arg(),
-                           wT_ + (size_t)m0 * M_, table() ? ew_.as<T>() + (size_t)m0 * M_ : nullptr, M_);
+                           wT_ + (size_t)m0 * M_, ew_.as<T>() + (size_t)m0 * M_, M_);
         FTS_HIP_CHECK(hipGetLastError());
     }
     for (int i = 0; i < n_qinit_; i++) {

@@ -1,0 +1,97 @@
+"""Sizes at the edges of the kernels that a grid's lengths choose, on the GPU against the oracle.
+
+One-dimensional grids: the direct convolution's lane and chunk counts change at 64 and 128 points and it ends
+at 256; longer ones take the generic kernels. Two-dimensional grids (one slab) run whole runs of steps in one
+launch. Real-space sweeps: lanes per line and the LDS pitch change at multiples of 16 and at 1024 points.
+
+Bars: FP64 1e-10 relative as in the other oracle tests; FP32 2e-5, the stated error of that form.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests.conftest import golden
+
+pytestmark = pytest.mark.gpu
+
+
+def say(msg):
+    print(msg, flush=True)
+
+
+def rel(a, b):
+    a, b = np.asarray(a), np.asarray(b)
+    return float(np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-300))
+
+
+@pytest.fixture(scope="module")
+def capi():
+    from langevin_fts_amd import capi as c
+    return c
+
+
+@pytest.fixture(scope="module")
+def ctx(capi):
+    return capi.Context(0)
+
+
+def check(ctx, capi, name, model, nx, prec="fp64", mask=None, bc=None, stress=True):
+    plan = golden("plans")[f"{name}|{model}|0"]
+    inp = plan["input"]
+    M = int(np.prod(nx))
+    rng = np.random.default_rng(23)
+    w = {m: 0.6 * rng.standard_normal(M) for m in inp["bonds"]}
+    # Real-space steps: a right side carries a rounding error of about 4 r eps of q, r = b^2 ds / (12 dx^2), which
+    # the solve passes on at long wavelengths. At 2.3 over 1023 points (r of 800 or more, some 100 steps) that
+    # alone is 1e-10 on Q, oracle included; at dx = 0.05 it is below 1e-12.
+    lx = [2.3 + 0.4 * i if bc is None else 0.05 * n for i, n in enumerate(nx)]
+    ref = O.Solver(O.Grid(nx, lx, mask), plan, inp["ds"], inp["bonds"], inp["solvents"], realspace_bc=bc)
+    ref.compute_statistics(w)
+    g = capi.Grid(ctx, nx, lx, mask)
+    P = capi.Plan(plan, inp["ds"], inp["bonds"], plan["schedules"]["4"], inp["solvents"])
+    s = capi.Solver(g, P, capi.FTS_FP64 if prec == "fp64" else capi.FTS_FP32, realspace_bc=bc)
+    bar = 1e-10 if prec == "fp64" else 2e-5
+    for again in range(2):
+        s.compute_statistics(w)
+        for p in range(len(plan["polymers"])):
+            assert abs(s.get_total_partition(p) / ref.get_total_partition(p) - 1) < bar
+        for m in inp["bonds"]:
+            assert rel(s.get_total_concentration(m), ref.get_total_concentration(m)) < bar
+    if stress and bc is None:
+        s.compute_stress()
+        ref.compute_stress()
+        assert rel(s.get_stress(), ref.get_stress()) < (bar if prec == "fp64" else 1e-4)
+
+
+MODELS = [("branched", "continuous"), ("diblock_f0.5_ds1_90", "discrete")]
+
+
+@pytest.mark.parametrize("name,model", MODELS)
+@pytest.mark.parametrize("n", [2, 30, 63, 64, 65, 126, 128, 130, 255, 256])
+def test_lines(ctx, capi, n, name, model):
+    say(f"line {n} {model}")
+    check(ctx, capi, name, model, [n])
+
+
+@pytest.mark.parametrize("name,model", MODELS)
+@pytest.mark.parametrize("nx", [[4, 4], [21, 26], [22, 35], [33, 64], [60, 104]])
+def test_flat_grids(ctx, capi, nx, name, model):
+    say(f"flat {nx} {model}")
+    rng = np.random.default_rng(4)
+    check(ctx, capi, name, model, nx)
+    check(ctx, capi, name, model, nx, mask=(rng.random(int(np.prod(nx))) > 0.1).astype(np.float64), stress=False)
+
+
+@pytest.mark.parametrize("nx", [[100], [45, 32], [27, 10, 16], [15, 18, 25]])
+def test_fp32(ctx, capi, nx):
+    say(f"fp32 {nx}")
+    check(ctx, capi, "diblock_f0.5_ds1_90", "discrete", nx, "fp32")
+
+
+@pytest.mark.parametrize("n", [15, 16, 17, 512, 1023, 1024, 1025])
+def test_realspace_lines(ctx, capi, n):
+    say(f"real-space sweeps {n}")
+    check(ctx, capi, "branched", "continuous", [n], bc=["periodic", "periodic"])
+    if n < 1000 or n == 1024:
+        check(ctx, capi, "branched", "continuous", [n, 3],
+              bc=["absorbing", "reflecting", "periodic", "periodic"])

@@ -320,7 +320,7 @@ def plan_dict(mol, an, model):
     return {"model": model, "polymers": pols, "propagators": props, "blocks": blocks}
 
 
-SLAB_KERNEL = re.compile(r"slab_kernel_\w+<double, 1, 64(, \d+)?>")
+SLAB_KERNEL = re.compile(r"slab_cube_kernel<double, 1, 64(, \d+)?>")
 
 
 def fft_schedule_info(n):
@@ -470,7 +470,7 @@ def replica_bench(args, w, lf, lfts):
     }
     if kern:
         out["roofline"] = kernel_roofline(
-            kern, f"slab pass (slab_kernel_wl<double, 1, {w['nx'][0]}, threads>: up to 32 propagators per launch)")
+            kern, f"slab pass (slab_cube_kernel<double, 1, {w['nx'][0]}, threads>: up to 32 propagators per launch)")
     print(json.dumps(out), flush=True)
 
 
@@ -1024,7 +1024,7 @@ def main():
         out["roofline"] = {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBPS, "unit": "GB/s",
                            "frac": achieved / PEAK_HBM_GBPS,
                            "traffic": traffic["bytes"] if traffic else None,
-                           "kernel": "slab pass (slab_kernel_wl<double, 1, 64, threads>: 2 propagators per "
+                           "kernel": "slab pass (slab_cube_kernel<double, 1, 64, threads>: 2 propagators per "
                                      "launch), timed in a pass of plain FP64 steps after the arms",
                            "timed_launch_count": sl["launches"],
                            "avg_launch_us": 1e3 * sl["milliseconds"] / max(sl["launches"], 1),

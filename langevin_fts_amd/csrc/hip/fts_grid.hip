@@ -306,7 +306,9 @@ void Grid::setup_fft() {
     sg.ay = ay;
     sg.az = az;
     sg.inv_m = 1.0 / (double)M;
-    slab_threads = choose_threads(sg.ny * sg.nz);
+    // the row split and merge hold SPLIT_MAXE values per thread and take a row at a time at least: up to
+    // 4096 points a row fits (one-dimensional grids above 256 points would else lose its end)
+    slab_threads = std::max(choose_threads(sg.ny * sg.nz), std::min(1024, ceil_div(ceil_div(sg.nz, SPLIT_MAXE), 64) * 64));
     const int per_thread = ceil_div(sg.ny * sg.nz, slab_threads);
     FTS_REQUIRE(per_thread <= 16, "y-z slab too large (more than 16384 points)");
     // the 8-value variant is compiled for at most 512 threads (more registers per thread)

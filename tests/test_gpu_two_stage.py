@@ -95,3 +95,11 @@ def test_realspace_lines(ctx, capi, n):
     if n < 1000 or n == 1024:
         check(ctx, capi, "branched", "continuous", [n, 3],
               bc=["absorbing", "reflecting", "periodic", "periodic"])
+
+
+@pytest.mark.parametrize("prec,n", [("fp64", 260), ("fp64", 512), ("fp64", 1001), ("fp64", 2187), ("fp32", 300)])
+def test_long_lines(ctx, capi, prec, n):
+    """One-dimensional grids beyond the direct convolution: a row of the slab pass must fit its threads."""
+    say(f"long line {n} {prec}")
+    for name, model in MODELS[1:] if prec == "fp32" else MODELS:
+        check(ctx, capi, name, model, [n], prec)

@@ -345,7 +345,7 @@ void Grid::setup_fft() {
         const int n = tnx[0];
         if (n == 32 || n == 48 || n == 64 || n == 96 || n == 128) ct_n = n;
     }
-    // wave-local line transforms for those grids (env FTS_CT_KERNELS=1: the block-synchronous ones)
+    // two-stage kernels of constant geometry for those grids (env FTS_CT_KERNELS=1: the block-synchronous ones)
     wave_local = ct_n != 0 && !std::getenv("FTS_CT_KERNELS");
     if (ct_n) set_lds_attributes_ct();
     if (wave_local) {
@@ -377,7 +377,7 @@ void Grid::setup_fft() {
 }
 
 // ------------------------------------------------------------------ FFT schedule autotuner
-// Times every pair of launch shapes of the wave-local slab and pencil kernels for this
+// Times every pair of launch shapes of the N^3 slab and pencil kernels for this
 // grid and precision on scratch fields (steps of two propagators: slab inverse+forward
 // with the exp(-w ds) factors, then the pencil pass with the bond factors, alternating
 // as in a propagator), and keeps the fastest pair; it replaces the defaults only when

@@ -97,7 +97,7 @@ public:
     double tdx[3];
     int M, nzc, Mc;
     // row pitch and per-field size (complex elements) of the half spectra in device
-    // buffers: nzc and Mc, or the padded pitch of the wave-local kernels
+    // buffers: nzc and Mc, or the padded pitch of the two-stage kernels
     int spitch = 0;     // FP64 spectrum row pitch (complex elements)
     int spitch32 = 0;   // FP32 spectrum row pitch
     size_t Ms = 0;      // spectrum slot (complex elements), for either precision
@@ -113,11 +113,11 @@ public:
     int slab_maxr = 8;   // real values per thread in the slab kernel (8 or 16)
     bool big = false;        // some axis needs a radix outside {2, 3, 4, 5, 8}
     int ct_n = 0;        // N of the compile-time specialised kernels for an N^3 grid, 0: runtime kernels
-    bool wave_local = false; // N^3 grids: one wavefront per line transform
+    bool wave_local = false; // N^3 grids with the two-stage kernels of constant geometry
     // other grids whose lengths all have a two-stage plan, per precision ([0] FP64, [1] FP32)
     bool two_stage[2] = {false, false};
     TwoGeom two[2];
-    // launch shapes of the wave-local kernels per precision ([0] FP64, [1] FP32):
+    // launch shapes of the N^3 kernels per precision ([0] FP64, [1] FP32):
     // slab workgroup size and pencil kz columns per wavefront, with how they were chosen
     int slab_bd[2] = {0, 0};
     // per slab mode (forward, half step, Richardson step): a workgroup size that

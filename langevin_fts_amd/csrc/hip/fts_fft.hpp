@@ -25,7 +25,10 @@ namespace fts {
 constexpr int FFT_MAX_STAGES = 12;
 constexpr int MAX_BATCH = 32;   // work items per launch (passed by value, kernel arguments < 4 KiB)
 constexpr int FFT_MAXE = 8;     // complex values held per thread per FFT stage
-constexpr int SPLIT_MAXE = 4;   // complex pairs held per thread in the real-row split/merge
+constexpr int SPLIT_MAXE = 4;   // complex pairs held per thread in the real-row split
+// complex values held per thread in the row merge, a whole row at a time at least: 1024 threads hold the
+// longest row that fits the LDS (5118 points in FP64: a packed row pair and the roots of unity)
+constexpr int MERGE_MAXE = 5;
 
 struct AxisPlan {
     int L;
@@ -74,6 +77,21 @@ inline int group_lines(const AxisPlan& p, int bd) {
     }
     FTS_REQUIRE(g >= 1, "FFT line of length " + std::to_string(p.L) + " does not fit the block");
     return g;
+}
+
+// ~8 elements per thread, whole waves, at most 1024 threads
+inline int choose_threads(int work) {
+    int bd = ceil_div(ceil_div(work, 8), 64) * 64;
+    return std::max(64, std::min(1024, bd));
+}
+
+// Threads of the generic slab kernel for ny rows of nz points: those of choose_threads, and at least as many as
+// hold one row in the split and the merge (one-dimensional grids above 256 points would else lose its end)
+inline int slab_block(int ny, int nz) {
+    const int bd = std::max(choose_threads(ny * nz), std::min(1024, ceil_div(ceil_div(nz, SPLIT_MAXE), 64) * 64));
+    FTS_REQUIRE(nz <= MERGE_MAXE * bd && nz / 2 + 1 <= SPLIT_MAXE * bd,
+                "rows of " + std::to_string(nz) + " points do not fit the block");
+    return bd;
 }
 
 // ------------------------------------------------------------------ complex helpers
@@ -333,7 +351,7 @@ __device__ void slab_forward_lds(T2* S, const SlabGeom& g, const T2* Wy, const T
     const int np = g.rows >> 1;
     lds_fft<-1, BIG, T>(S, np, 2 * g.P, 1, g.az, Wz);
     // split: X_a[k] = (Z[k] + conj Z[-k]) / 2, X_b[k] = -i (Z[k] - conj Z[-k]) / 2;
-    // pairs are independent, processed in groups that fit FFT_MAXE values per thread
+    // pairs are independent, processed in groups that fit SPLIT_MAXE pairs per thread
     const int pg = max(1, (SPLIT_MAXE * (int)blockDim.x) / g.nzc);
     for (int p0 = 0; p0 < np; p0 += pg) {
         const int total = min(pg, np - p0) * g.nzc;
@@ -371,12 +389,12 @@ template <bool BIG, typename T, typename T2>
 __device__ void slab_inverse_lds(T2* S, const SlabGeom& g, const T2* Wy, const T2* Wz) {
     lds_fft<+1, BIG, T>(S, g.nzc, 1, g.P, g.ay, Wy);
     const int np = g.rows >> 1;
-    const int pg = max(1, (SPLIT_MAXE * (int)blockDim.x) / g.nz);
+    const int pg = max(1, (MERGE_MAXE * (int)blockDim.x) / g.nz);
     for (int p0 = 0; p0 < np; p0 += pg) {
         const int total = min(pg, np - p0) * g.nz;
-        T2 vz[SPLIT_MAXE];
+        T2 vz[MERGE_MAXE];
 #pragma unroll
-        for (int t = 0; t < SPLIT_MAXE; t++) {
+        for (int t = 0; t < MERGE_MAXE; t++) {
             const int f = threadIdx.x + t * blockDim.x;
             if (f < total) {
                 const int p = p0 + f / g.nz, k = f % g.nz;
@@ -398,7 +416,7 @@ __device__ void slab_inverse_lds(T2* S, const SlabGeom& g, const T2* Wy, const T
         }
         __syncthreads();
 #pragma unroll
-        for (int t = 0; t < SPLIT_MAXE; t++) {
+        for (int t = 0; t < MERGE_MAXE; t++) {
             const int f = threadIdx.x + t * blockDim.x;
             if (f < total) {
                 const int p = p0 + f / g.nz, k = f % g.nz;

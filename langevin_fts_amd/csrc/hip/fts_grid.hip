@@ -79,12 +79,6 @@ fts_kernel_stats KernelTimer::get(int family) {
 
 namespace {
 
-// ~8 elements per thread, whole waves, at most 1024 threads
-int choose_threads(int work) {
-    int bd = ceil_div(ceil_div(work, 8), 64) * 64;
-    return std::max(64, std::min(1024, bd));
-}
-
 template <typename T>
 void upload_twiddles(int L, DeviceBuffer& buf) {
     using T2 = typename vec2<T>::type;
@@ -306,9 +300,7 @@ void Grid::setup_fft() {
     sg.ay = ay;
     sg.az = az;
     sg.inv_m = 1.0 / (double)M;
-    // the row split and merge hold SPLIT_MAXE values per thread and take a row at a time at least: up to
-    // 4096 points a row fits (one-dimensional grids above 256 points would else lose its end)
-    slab_threads = std::max(choose_threads(sg.ny * sg.nz), std::min(1024, ceil_div(ceil_div(sg.nz, SPLIT_MAXE), 64) * 64));
+    slab_threads = slab_block(sg.ny, sg.nz);
     const int per_thread = ceil_div(sg.ny * sg.nz, slab_threads);
     FTS_REQUIRE(per_thread <= 16, "y-z slab too large (more than 16384 points)");
     // the 8-value variant is compiled for at most 512 threads (more registers per thread)

@@ -121,12 +121,6 @@ void run_grid(dim3 grid, dim3 block, size_t lds, F&& kernel) {
         }
 }
 
-// Grid::setup_fft's choice of workgroup size: about 8 elements per thread, whole waves
-int choose_threads(int work) {
-    int bd = fts::ceil_div(fts::ceil_div(work, 8), 64) * 64;
-    return std::max(64, std::min(1024, bd));
-}
-
 template <typename T>
 std::vector<typename fts::vec2<T>::type> twiddles(int L) {
     std::vector<typename fts::vec2<T>::type> h(L);
@@ -163,7 +157,7 @@ int run(const char* pass, const char* dir, const int* n, const char* in_path, co
         g.ay = ay;
         g.az = az;
         g.inv_m = 1.0 / (double)M;
-        const int threads = choose_threads(ny * nz);
+        const int threads = fts::slab_block(ny, nz);
         const int per_thread = fts::ceil_div(ny * nz, threads);
         const int maxr = (per_thread <= 8 && threads <= 512) ? 8 : 16;
         g.ay.group = fts::group_lines(g.ay, threads);
@@ -209,7 +203,7 @@ int run(const char* pass, const char* dir, const int* n, const char* in_path, co
         g.n_tiles = tiles;
         g.P = C;
         g.ax = ax;
-        const int threads = choose_threads(nx * C);
+        const int threads = fts::choose_threads(nx * C);
         g.ax.group = fts::group_lines(g.ax, threads);
         const size_t lds = (size_t)(nx * g.P + nx) * sizeof(T2);
         std::printf("xpass: threads %d, tile %d x %d, big %d, x group %d, lds %zu\n", threads, C, tiles, big,

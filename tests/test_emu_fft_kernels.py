@@ -64,7 +64,11 @@ def run(exe, kind, direction, esize, n, a, tmp):
     return np.fromfile(fo, dtype=a.dtype), r.stdout
 
 
-@pytest.mark.parametrize("n,esize", [((7, 11, 13), 4), ((7, 11, 13), 8), ((13, 6, 10), 4), ((5, 4, 3), 4)])
+# rows of more than 4 values per thread of the largest workgroup; the longest that the LDS takes have 5118 points
+LONG_ROWS = [((1, 1, 5115), 8), ((1, 2, 5000), 8)]
+
+
+@pytest.mark.parametrize("n,esize", [((7, 11, 13), 4), ((7, 11, 13), 8), ((13, 6, 10), 4), ((5, 4, 3), 4)] + LONG_ROWS)
 def test_emulated_kernels_transform_correctly(tmp_path, n, esize):
     tmp = str(tmp_path)
     dt = np.float32 if esize == 4 else np.float64

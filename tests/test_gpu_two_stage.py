@@ -97,9 +97,26 @@ def test_realspace_lines(ctx, capi, n):
               bc=["absorbing", "reflecting", "periodic", "periodic"])
 
 
-@pytest.mark.parametrize("prec,n", [("fp64", 260), ("fp64", 512), ("fp64", 1001), ("fp64", 2187), ("fp32", 300)])
+@pytest.mark.parametrize("prec,n", [("fp64", 260), ("fp64", 512), ("fp64", 1001), ("fp64", 2187), ("fp32", 300),
+                                    ("fp64", 4096), ("fp64", 4500)])
 def test_long_lines(ctx, capi, prec, n):
     """One-dimensional grids beyond the direct convolution: a row of the slab pass must fit its threads."""
     say(f"long line {n} {prec}")
     for name, model in MODELS[1:] if prec == "fp32" else MODELS:
         check(ctx, capi, name, model, [n], prec)
+
+
+def test_two_long_rows(ctx, capi):
+    say("2 x 5000")
+    check(ctx, capi, *MODELS[1], [2, 5000])
+
+
+def test_rows_beyond_the_lds_are_refused(ctx, capi):
+    """A line of 5120 points has no slab plan: the pseudo-spectral solver says so, real-space steps take it."""
+    plan = golden("plans")["diblock_f0.5_ds1_16|continuous|0"]
+    inp = plan["input"]
+    g = capi.Grid(ctx, [5120], [6.0])
+    P = capi.Plan(plan, inp["ds"], inp["bonds"], plan["schedules"]["4"])
+    with pytest.raises(RuntimeError, match="LDS"):
+        capi.Solver(g, P)
+    capi.Solver(g, P, realspace_bc=["periodic", "periodic"])

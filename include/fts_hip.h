@@ -80,7 +80,9 @@ int fts_grid_inner_product(fts_grid* g, const double* a, const double* b, int on
  * backward (MklFFT3D.cpp:55-79): forward unnormalised real -> half complex
  * [nx][ny][nz/2+1] (interleaved re,im), backward half complex -> real divided by
  * the grid size. precision FTS_FP64 (double) or FTS_FP32 (float). In-place is not
- * allowed. batch fields are contiguous. */
+ * allowed. batch fields are contiguous. Both return when the transforms are done.
+ * Backward transforms, and forward ones on the N^3 grids named below, allocate a
+ * workspace for the call. */
 int fts_grid_fft_forward(fts_grid* g, int precision, const void* d_in, void* d_out, int batch);
 int fts_grid_fft_backward(fts_grid* g, int precision, const void* d_in, void* d_out, int batch);
 /* No counterpart in the reference: fts_grid_fft_backward for callers that cannot
@@ -88,8 +90,9 @@ int fts_grid_fft_backward(fts_grid* g, int precision, const void* d_in, void* d_
  * that forbid hipMalloc). Same arguments and results (bit for bit); it allocates
  * nothing and does not synchronise: the work is enqueued on the context's stream.
  * Its workspace is a fixed 32 MiB array per GPU, kept until the process ends: a grid
- * whose half spectrum (nx ny (nz/2+1) rounded up to rows of 8, times 16 bytes in
- * FP64, 8 in FP32) exceeds it is refused with an error (128^3 FP64 needs 18.9 MB).
+ * whose half spectrum (nx ny (nz/2+1) values of 16 bytes in FP64, 8 in FP32; rows of
+ * the N^3 grids named below rounded up to 128 bytes) exceeds it is refused with an
+ * error (128^3 FP64 needs 18.9 MB).
  * Every call on one GPU shares that array, so calls whose work overlaps on one GPU
  * (other streams or contexts on the device) race; calls in one stream do not. */
 int fts_grid_fft_backward_noalloc(fts_grid* g, int precision, const void* d_in, void* d_out, int batch);

@@ -635,7 +635,7 @@ static double slab_bytes(const Grid& g, int mode, const SlabBatch<T>& b) {
 }
 
 template <typename T>
-void Grid::launch_slab(int mode, const SlabBatch<T>& b) const {
+void Grid::launch_slab(int mode, const SlabBatch<T>& b, bool contiguous) const {
     require_supported<T>(*this);
     if (b.n == 0) return;
     KernelTimer& timer = ctx->timer;
@@ -648,7 +648,7 @@ void Grid::launch_slab(int mode, const SlabBatch<T>& b) const {
         case 128: launch_slab_ct<T, 128>(*this, mode, b); break;
         default: {
             if (two_stage[prec_index<T>()]) {
-                launch_slab_two<T>(mode, b);
+                launch_slab_two<T>(mode, b, contiguous);
                 break;
             }
             const dim3 grid(tnx[0], b.n), block(slab_threads);
@@ -663,7 +663,7 @@ void Grid::launch_slab(int mode, const SlabBatch<T>& b) const {
 }
 
 template <typename T>
-void Grid::launch_xpass(const XBatch<T>& b, const T* bx, const T* by, const T* bz) const {
+void Grid::launch_xpass(const XBatch<T>& b, const T* bx, const T* by, const T* bz, bool contiguous) const {
     require_supported<T>(*this);
     if (b.n == 0) return;
     if (tnx[0] == 1 && bx == nullptr) return;   // a transform of length 1
@@ -677,7 +677,7 @@ void Grid::launch_xpass(const XBatch<T>& b, const T* bx, const T* by, const T* b
         case 128: launch_xpass_ct<T, 128>(*this, b, bx, by, bz); break;
         default: {
             if (two_stage[prec_index<T>()]) {
-                launch_xpass_two<T>(b, bx, by, bz);
+                launch_xpass_two<T>(b, bx, by, bz, contiguous);
                 break;
             }
             const dim3 grid(tnx[1] * xg.n_tiles, b.n), block(x_threads);
@@ -766,28 +766,30 @@ template <typename T>
 void Grid::fft_forward(const T* in, typename vec2<T>::type* out, int batch) {
     require_fft();
     using T2 = typename vec2<T>::type;
-    // padded rows: transform into a workspace of the padded layout, then copy the rows out
-    const int pitch = spec_pitch<T>();
+    // the N^3 kernels are compiled for padded rows: transform into a workspace of that layout, then copy
+    // the rows out; the others write the caller's rows
+    const int pitch = fft_pitch<T>();
     const bool padded = pitch != nzc;
     DeviceBuffer tmp;
-    if (padded) tmp.allocate(sizeof(T2) * Ms * std::min(batch, MAX_BATCH));
+    const size_t slot = fft_slot<T>();
+    if (padded) tmp.allocate(sizeof(T2) * slot * std::min(batch, MAX_BATCH));
     for (int b0 = 0; b0 < batch; b0 += MAX_BATCH) {
         const int nb = std::min(MAX_BATCH, batch - b0);
         SlabBatch<T> sb{};
         XBatch<T> xb{};
         sb.n = xb.n = nb;
         for (int b = 0; b < nb; b++) {
-            T2* spec = padded ? tmp.as<T2>() + (size_t)b * Ms : out + (size_t)(b0 + b) * Mc;
+            T2* spec = padded ? tmp.as<T2>() + (size_t)b * slot : out + (size_t)(b0 + b) * Mc;
             SlabItem<T>& it = sb.it[b];
             it.qin = in + (size_t)(b0 + b) * M;
             it.c0 = spec;
             it.n_out = 1;
             xb.it[b] = XItem<T>{spec, -1};
         }
-        launch_slab<T>(SLAB_FWD, sb);
-        launch_xpass<T>(xb, nullptr, nullptr, nullptr);
+        launch_slab<T>(SLAB_FWD, sb, true);
+        launch_xpass<T>(xb, nullptr, nullptr, nullptr, true);
         for (int b = 0; padded && b < nb; b++)
-            FTS_HIP_CHECK(hipMemcpy2DAsync(out + (size_t)(b0 + b) * Mc, sizeof(T2) * nzc, tmp.as<T2>() + (size_t)b * Ms,
+            FTS_HIP_CHECK(hipMemcpy2DAsync(out + (size_t)(b0 + b) * Mc, sizeof(T2) * nzc, tmp.as<T2>() + (size_t)b * slot,
                                            sizeof(T2) * pitch, sizeof(T2) * nzc, (size_t)tnx[0] * tnx[1],
                                            hipMemcpyDeviceToDevice, stream()));
     }
@@ -799,29 +801,29 @@ void Grid::fft_backward_ws(const typename vec2<T>::type* in, T* out, int batch, 
                            int ws_fields) {
     require_fft();
     // the pencil pass transforms in place, so the input is first copied into the
-    // workspace (ws_fields spectra of Ms elements), in chunks of at most ws_fields
+    // workspace (ws_fields spectra of fft_slot elements), in chunks of at most ws_fields
     using T2 = typename vec2<T>::type;
     FTS_REQUIRE(ws_fields >= 1, "the FFT workspace holds no spectrum");
     const int chunk = std::min(ws_fields, MAX_BATCH);
+    const size_t slot = fft_slot<T>();
     for (int b0 = 0; b0 < batch; b0 += chunk) {
         const int nb = std::min(chunk, batch - b0);
-        // the caller's rows of nzc values into the workspace's rows of this precision's
-        // pitch, one spectrum per slot of Ms elements (Ms fits the wider pitch of the two)
+        // the caller's rows of nzc values into the rows that the kernels read
         for (int b = 0; b < nb; b++)
-            FTS_HIP_CHECK(hipMemcpy2DAsync(ws + (size_t)b * Ms, sizeof(T2) * spec_pitch<T>(),
+            FTS_HIP_CHECK(hipMemcpy2DAsync(ws + (size_t)b * slot, sizeof(T2) * fft_pitch<T>(),
                                            in + (size_t)(b0 + b) * Mc, sizeof(T2) * nzc, sizeof(T2) * nzc,
                                            (size_t)tnx[0] * tnx[1], hipMemcpyDeviceToDevice, stream()));
         SlabBatch<T> sb{};
         XBatch<T> xb{};
         sb.n = xb.n = nb;
         for (int b = 0; b < nb; b++) {
-            xb.it[b] = XItem<T>{ws + (size_t)b * Ms, -2};
+            xb.it[b] = XItem<T>{ws + (size_t)b * slot, -2};
             SlabItem<T>& it = sb.it[b];
-            it.c0 = ws + (size_t)b * Ms;
+            it.c0 = ws + (size_t)b * slot;
             it.qout = out + (size_t)(b0 + b) * M;
         }
-        launch_xpass<T>(xb, nullptr, nullptr, nullptr);
-        launch_slab<T>(SLAB_INV1, sb);
+        launch_xpass<T>(xb, nullptr, nullptr, nullptr, true);
+        launch_slab<T>(SLAB_INV1, sb, true);
     }
 }
 
@@ -830,7 +832,7 @@ void Grid::fft_backward(const typename vec2<T>::type* in, T* out, int batch) {
     require_fft();
     using T2 = typename vec2<T>::type;
     const int nw = std::min(batch, MAX_BATCH);
-    DeviceBuffer tmp(sizeof(T2) * Ms * nw);
+    DeviceBuffer tmp(sizeof(T2) * fft_slot<T>() * nw);
     fft_backward_ws<T>(in, out, batch, tmp.as<T2>(), nw);
     FTS_HIP_CHECK(hipStreamSynchronize(stream()));
 }
@@ -872,7 +874,7 @@ void Grid::fft_backward_noalloc(const typename vec2<T>::type* in, T* out, int ba
         ws = ctx->device >= 0 && ctx->device < MAX_DEVICES ? scratch_ptr[ctx->device] : nullptr;
     }
     FTS_REQUIRE(ws != nullptr, "the no-allocation workspace of this device is not set up");
-    const size_t per_field = sizeof(T2) * Ms;
+    const size_t per_field = sizeof(T2) * fft_slot<T>();
     if (per_field > NOALLOC_SCRATCH_BYTES)
         throw Error("fts_grid_fft_backward_noalloc: one spectrum of this grid takes " + std::to_string(per_field) +
                     " bytes of workspace; the no-allocation workspace holds " +
@@ -880,10 +882,9 @@ void Grid::fft_backward_noalloc(const typename vec2<T>::type* in, T* out, int ba
     fft_backward_ws<T>(in, out, batch, static_cast<T2*>(ws), (int)(NOALLOC_SCRATCH_BYTES / per_field));
 }
 
-template void Grid::launch_slab<double>(int, const SlabBatch<double>&) const;
-template void Grid::launch_slab<float>(int, const SlabBatch<float>&) const;
-template void Grid::launch_xpass<double>(const XBatch<double>&, const double*, const double*, const double*) const;
-template void Grid::launch_xpass<float>(const XBatch<float>&, const float*, const float*, const float*) const;
+template void Grid::launch_slab<double>(int, const SlabBatch<double>&, bool) const;
+template void Grid::launch_slab<float>(int, const SlabBatch<float>&, bool) const;
+template void Grid::launch_xpass<double>(const XBatch<double>&, const double*, const double*, const double*, bool) const;
 template int Grid::launch_stress_pencil<double>(const StressBatch<double>&, const StressGeom&, const double*,
                                                 const double*, const double*, double*) const;
 template int Grid::launch_stress_pencil<float>(const StressBatch<float>&, const StressGeom&, const float*,

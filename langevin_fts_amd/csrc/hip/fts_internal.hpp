@@ -144,6 +144,16 @@ public:
     int spec_pitch() const {
         return sizeof(T) == sizeof(float) ? spitch32 : spitch;
     }
+    // rows and size (complex elements) of a spectrum in the public transforms: the caller's contiguous layout,
+    // but for the N^3 kernels, which are compiled for padded rows
+    template <typename T>
+    int fft_pitch() const {
+        return wave_local ? spec_pitch<T>() : nzc;
+    }
+    template <typename T>
+    size_t fft_slot() const {
+        return (size_t)tnx[0] * tnx[1] * fft_pitch<T>();
+    }
     template <typename T>
     const T* mask() const;
     template <typename T>
@@ -156,10 +166,11 @@ public:
     size_t x_lds() const {
         return (size_t)(xg.nx * xg.P + xg.nx) * sizeof(typename vec2<T>::type);
     }
+    // contiguous: spectra in rows of fft_pitch values, not spec_pitch
     template <typename T>
-    void launch_slab(int mode, const SlabBatch<T>& b) const;
+    void launch_slab(int mode, const SlabBatch<T>& b, bool contiguous = false) const;
     template <typename T>
-    void launch_xpass(const XBatch<T>& b, const T* bx, const T* by, const T* bz) const;
+    void launch_xpass(const XBatch<T>& b, const T* bx, const T* by, const T* bz, bool contiguous = false) const;
     // Grids of one x-slab with a two-stage plan: whole runs of steps in one launch. by, bz: bond tables.
     template <typename T>
     bool flat() const {
@@ -168,9 +179,9 @@ public:
     template <typename T>
     void launch_flat(bool continuous, const FlatBatch<T>& b, const T* by, const T* bz) const;
     template <typename T>
-    void launch_slab_two(int mode, const SlabBatch<T>& b) const;
+    void launch_slab_two(int mode, const SlabBatch<T>& b, bool contiguous) const;
     template <typename T>
-    void launch_xpass_two(const XBatch<T>& b, const T* bx, const T* by, const T* bz) const;
+    void launch_xpass_two(const XBatch<T>& b, const T* bx, const T* by, const T* bz, bool contiguous) const;
     // The stress of b.n terms from the slab pass's output spectra, with their x transforms
     // fused into the reduction (wave-local grids only): 3 partial sums per workgroup into
     // partials, term-major; returns the workgroups per term.
@@ -188,8 +199,8 @@ public:
     void fft_forward(const T* in, typename vec2<T>::type* out, int batch);
     template <typename T>
     void fft_backward(const typename vec2<T>::type* in, T* out, int batch);
-    // fft_backward through a caller's workspace of ws_fields spectra (Ms elements
-    // each): enqueued on the stream, no allocation, no synchronisation
+    // fft_backward through a caller's workspace of ws_fields spectra (fft_slot
+    // elements each): enqueued on the stream, no allocation, no synchronisation
     template <typename T>
     void fft_backward_ws(const typename vec2<T>::type* in, T* out, int batch, typename vec2<T>::type* ws,
                          int ws_fields);

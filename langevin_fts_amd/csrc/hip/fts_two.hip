@@ -16,6 +16,12 @@ template <typename T>
 constexpr int prec() {
     return sizeof(T) == sizeof(float) ? 1 : 0;
 }
+
+// the plan for spectra of the grid's padded rows, or of rows of nzc values (a caller's layout)
+TwoGeom two_rows(TwoGeom t, bool contiguous) {
+    if (contiguous) t.sp = t.nzc;
+    return t;
+}
 }  // namespace
 
 template <typename T>
@@ -30,18 +36,18 @@ void two_set_lds_limits() {
 }
 
 template <typename T>
-void Grid::launch_slab_two(int mode, const SlabBatch<T>& b) const {
+void Grid::launch_slab_two(int mode, const SlabBatch<T>& b, bool contiguous) const {
     // the first half step of a Richardson pair waits in the output slice
     for (int i = 0; i < b.n; i++)
         if (mode == SLAB_INV2 && !b.it[i].qout) throw Error("slab item without the real slice its second pass reads");
-    const TwoGeom& t = two[prec<T>()];
+    const TwoGeom t = two_rows(two[prec<T>()], contiguous);
     hipLaunchKernelGGL((slab_two_kernel<T>), dim3(tnx[0], b.n), dim3(two_slab_threads(t)),
                        two_slab_lds(t, sizeof(typename vec2<T>::type)), stream(), t, mode, b, tw<T>(1), tw<T>(2));
 }
 
 template <typename T>
-void Grid::launch_xpass_two(const XBatch<T>& b, const T* bx, const T* by, const T* bz) const {
-    const TwoGeom& t = two[prec<T>()];
+void Grid::launch_xpass_two(const XBatch<T>& b, const T* bx, const T* by, const T* bz, bool contiguous) const {
+    const TwoGeom t = two_rows(two[prec<T>()], contiguous);
     constexpr int e = sizeof(typename vec2<T>::type);
     const int tiles = ceil_div(t.nzc, two_pencil_columns(e));
     hipLaunchKernelGGL((pencil_two_kernel<T>), dim3(tnx[1] * tiles, b.n), dim3(64), two_pencil_lds(t, two_pencil_columns(e), e), stream(), t,
@@ -81,8 +87,8 @@ void Grid::launch_flat(bool continuous, const FlatBatch<T>& b, const T* by, cons
 
 #define FTS_TWO_INSTANCES(T)                                                                        \
     template void two_set_lds_limits<T>();                                                          \
-    template void Grid::launch_slab_two<T>(int, const SlabBatch<T>&) const;                         \
-    template void Grid::launch_xpass_two<T>(const XBatch<T>&, const T*, const T*, const T*) const;  \
+    template void Grid::launch_slab_two<T>(int, const SlabBatch<T>&, bool) const;                   \
+    template void Grid::launch_xpass_two<T>(const XBatch<T>&, const T*, const T*, const T*, bool) const; \
     template void Grid::launch_flat<T>(bool, const FlatBatch<T>&, const T*, const T*) const;
 FTS_TWO_INSTANCES(double)
 FTS_TWO_INSTANCES(float)

@@ -249,7 +249,6 @@ Grid::Grid(fts_context* c, int d, const int* n, const double* l, const double* m
     nzc = tnx[2] / 2 + 1;
     Mc = tnx[0] * tnx[1] * nzc;
     spitch = spitch32 = nzc;
-    Ms = (size_t)Mc;
     // ComputationBox.cpp:47-98: dv = prod dx (times mask), volume = prod lx
     dV = 1.0;
     for (int i = 0; i < dim; i++) dV *= dx[i];
@@ -343,7 +342,6 @@ void Grid::setup_fft() {
     if (wave_local) {
         spitch = wspec_pitch<vec2<double>::type>(ct_n);
         spitch32 = wspec_pitch<vec2<float>::type>(ct_n);
-        Ms = (size_t)tnx[0] * tnx[1] * std::max(spitch, spitch32);
         tune_fft_schedule<double>();
         tune_fft_schedule<float>();
     }
@@ -364,7 +362,6 @@ void Grid::setup_fft() {
             spitch32 = two[1].sp;
             two_set_lds_limits<float>();
         }
-        Ms = (size_t)tnx[0] * tnx[1] * std::max(spitch, spitch32);
     }
 }
 

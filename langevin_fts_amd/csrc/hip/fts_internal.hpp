@@ -96,11 +96,10 @@ public:
     int tnx[3];     // 3D-mapped sizes (Pseudo.cpp:31-45)
     double tdx[3];
     int M, nzc, Mc;
-    // row pitch and per-field size (complex elements) of the half spectra in device
-    // buffers: nzc and Mc, or the padded pitch of the two-stage kernels
+    // row pitch (complex elements) of the half spectra in device buffers: nzc, or the
+    // padded pitch of the two-stage kernels, whole 128-byte lines
     int spitch = 0;     // FP64 spectrum row pitch (complex elements)
     int spitch32 = 0;   // FP32 spectrum row pitch
-    size_t Ms = 0;      // spectrum slot (complex elements), for either precision
     double volume;
     double dV;
     std::vector<double> mask_h;
@@ -143,6 +142,11 @@ public:
     template <typename T>
     int spec_pitch() const {
         return sizeof(T) == sizeof(float) ? spitch32 : spitch;
+    }
+    // size of a spectrum in rows of spec_pitch
+    template <typename T>
+    size_t spec_slot() const {
+        return (size_t)tnx[0] * tnx[1] * spec_pitch<T>();
     }
     // rows and size (complex elements) of a spectrum in the public transforms: the caller's contiguous layout,
     // but for the N^3 kernels, which are compiled for padded rows

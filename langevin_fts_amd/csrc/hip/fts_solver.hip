@@ -142,7 +142,7 @@ private:
     int model_;
     double ds_;
     int M_;
-    size_t Ms_;   // spectrum workspace slot size (the grid's padded layout)
+    size_t Ms_;   // spectrum workspace slot size (the grid's padded layout at this precision)
     int n_mon_, n_qinit_;
     std::vector<double> bsq_;
     std::vector<Prop> props_;
@@ -201,7 +201,7 @@ Solver<T>::Solver(Grid* grid, const fts_plan* pl, const int* bc, bool reduce_mem
     }
     ds_ = pl->ds;
     M_ = g_->M;
-    Ms_ = g_->Ms;
+    Ms_ = g_->spec_slot<T>();
     n_mon_ = pl->n_monomers;
     n_qinit_ = pl->n_qinit;
     FTS_REQUIRE(model_ == FTS_CONTINUOUS || model_ == FTS_DISCRETE, "invalid chain model");
@@ -277,8 +277,10 @@ Solver<T>::Solver(Grid* grid, const fts_plan* pl, const int* bc, bool reduce_mem
     ew_.allocate(sizeof(T) * n_mon_ * (size_t)M_);
     if (n_qinit_) qinit_.allocate(sizeof(double) * n_qinit_ * (size_t)M_);
     // at least 8 stress terms per chunk, and 32 where their spectra stay below 64 MB: a chunk of
-    // a small grid is bound by its launches (128 points: 13 chunks took 270 us of an evaluation)
-    n_ws_ = std::max<int>(2 * (int)jmax, sizeof(T2) * 2 * MAX_BATCH * Ms_ <= ((size_t)64 << 20) ? 2 * MAX_BATCH : 16);
+    // a small grid is bound by its launches (128 points: 13 chunks took 270 us of an evaluation);
+    // real-space steps have no stress
+    const bool many = !real_ && sizeof(T2) * 2 * MAX_BATCH * Ms_ <= ((size_t)64 << 20);
+    n_ws_ = std::max<int>(2 * (int)jmax, many ? 2 * MAX_BATCH : 16);
     ws_.allocate(sizeof(T2) * (size_t)n_ws_ * Ms_);
     phib_.allocate(sizeof(double) * blocks_.size() * (size_t)M_);
     if (!svf_.empty()) phis_.allocate(sizeof(double) * svf_.size() * (size_t)M_);

@@ -253,3 +253,30 @@ def test_anderson_mixing_matches_reference(ctx, capi, name):
         wn = am.calculate_new_fields(w, d, old, err)
         np.testing.assert_allclose(wn, step["w_new"], rtol=0, atol=1e-10)
         w = np.array(step["w_new"])
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("nx", [[60, 64, 32], [32, 32, 32]])
+def test_workspace_is_sized_for_its_precision(ctx, capi, nx, prec):
+    """The solver's spectra have rows of whole 128-byte lines of their own precision: 24 values of 16 bytes for the 17
+    of nz = 32 in FP64, 32 values of 8 bytes in FP32, and no more than 64 of them."""
+    import ctypes
+
+    name = "diblock_f0.5_ds1_16|continuous|0"
+    plan = golden("plans")[name]
+    inp = plan["input"]
+    M = int(np.prod(nx))
+    e = 8 if prec == "fp64" else 4
+    say(f"workspace {nx} {prec}")
+    g = capi.Grid(ctx, nx, [4.0, 3.5, 3.0])
+    s = capi.Solver(g, capi.Plan(plan, inp["ds"], inp["bonds"], plan["schedules"]["4"]),
+                    capi.FTS_FP64 if prec == "fp64" else capi.FTS_FP32)
+    dev, host = ctypes.c_size_t(), ctypes.c_size_t()
+    capi.check(capi.lib().fts_solver_get_memory_usage(s.h, ctypes.byref(dev), ctypes.byref(host)))
+    slices = sum(p["max_n_segment"] + 1 for p in plan["propagators"])
+    mons = len(inp["bonds"])
+    fields = slices * e + mons * (8 + e + (4 if e == 4 else 0)) + 8 * len(plan["blocks"])
+    slot = 2 * e * nx[0] * nx[1] * (24 if e == 8 else 32)
+    terms = 64 if 64 * slot <= 64 << 20 else 16
+    assert dev.value - fields * M - terms * slot in range(0, 1 << 16)
+    assert host.value == 0

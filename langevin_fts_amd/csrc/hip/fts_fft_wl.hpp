@@ -116,21 +116,6 @@ __device__ __forceinline__ void wl_stages(typename WRegs<T2, L, REV, S, NLW, LF>
     }
 }
 
-// Row pitch (complex elements T2) of the half spectra that the wave-local passes exchange
-// through HBM: nz/2+1 rounded up to a whole number of 128-byte lines (8 columns in FP64,
-// 16 in FP32), so that every spectrum row, and with it every pencil tile of that many
-// columns, starts on a line. A tile that straddles two lines, or shares one with a
-// neighbouring tile on another XCD (its own L2), fetches lines twice. The pad columns are
-// never read or written. FTS_SPEC_PAD=0 (a tuning define) keeps nz/2+1.
-#ifndef FTS_SPEC_PAD
-#define FTS_SPEC_PAD 1
-#endif
-template <typename T2>
-constexpr int wspec_pitch(int N) {
-    constexpr int L = 128 / (int)sizeof(T2);
-    return FTS_SPEC_PAD ? (N / 2 + 1 + L - 1) / L * L : N / 2 + 1;
-}
-
 // ------------------------------------------------------------------ pencils of the stress pass
 template <int N, int NL_>
 struct WPencil {

@@ -340,8 +340,8 @@ void Grid::setup_fft() {
     wave_local = ct_n != 0 && !std::getenv("FTS_CT_KERNELS");
     if (ct_n) set_lds_attributes_ct();
     if (wave_local) {
-        spitch = wspec_pitch<vec2<double>::type>(ct_n);
-        spitch32 = wspec_pitch<vec2<float>::type>(ct_n);
+        spitch = two_pitch(nzc, sizeof(double2));
+        spitch32 = two_pitch(nzc, sizeof(float2));
         tune_fft_schedule<double>();
         tune_fft_schedule<float>();
     }
@@ -421,7 +421,7 @@ template <typename T, int N>
 TuneChoice tune_wave_local(const Grid& g) {
     using T2 = typename vec2<T>::type;
     constexpr int NZC = N / 2 + 1, ITEMS = 2;
-    const size_t M = (size_t)N * N * N, Mc = (size_t)N * N * wspec_pitch<T2>(N);
+    const size_t M = (size_t)N * N * N, Mc = (size_t)N * N * TwoCube<N, sizeof(T2)>::sp;
     DeviceBuffer spec, q, w, tab;
     // two spectra per item (c0, c1: the Richardson step and the two-spectrum forward
     // transform of continuous chains) and one real slice (qin and qout)

@@ -73,6 +73,15 @@ constexpr int two_conflicts(const TwoGeom& g, int pitch, int row) {
     return total;
 }
 
+// Row pitch (complex elements) of the half spectra that the passes exchange through HBM: nzc rounded up to a
+// whole number of 128-byte lines (8 columns in FP64, 16 in FP32), so that every row, and with it every
+// pencil tile of that many columns, starts on a line. A tile that straddles two lines, or shares one with a
+// neighbouring tile on another XCD (its own L2), fetches lines twice. The pad columns are never read
+// or written.
+constexpr int two_pitch(int nzc, int elem_bytes) {
+    const int line = 128 / elem_bytes;
+    return (nzc + line - 1) / line * line;
+}
 // The geometry of an nx x ny x nz grid, or false when a length has no plan or a plane does not
 // fit the LDS
 constexpr size_t two_slab_lds(const TwoGeom& g, int elem_bytes) {
@@ -85,8 +94,7 @@ constexpr bool two_geometry(const int* n, int elem_bytes, size_t lds_limit, TwoG
         return false;
     g.nx = n[0];
     g.nzc = n[2] / 2 + 1;
-    const int line = 128 / elem_bytes;
-    g.sp = (g.nzc + line - 1) / line * line;
+    g.sp = two_pitch(g.nzc, elem_bytes);
     g.lines = (g.y.r1 + 1) / 2 * g.y.r2;
     g.pad = g.z.r1 % 2 == 0 ? 1 : 0;
     const int row = 256 / elem_bytes, least = n[2] + g.pad * g.z.r2 + 2;

@@ -41,3 +41,13 @@ def test_null_arguments_are_errors_not_crashes():
     assert lib.fts_grid_set_lx(None, None) != 0
     assert b"null" in lib.fts_last_error()
     assert lib.fts_solver_compute_concentrations(None) != 0
+
+
+def test_no_build_define_changes_a_layout():
+    """FTS_HIP_DEFINES reaches every source: a header value that such a define replaces can differ between kernels that
+    share a buffer (a row pitch did). The emulators' hook for the LDS pointer is the only overridable name."""
+    src = os.path.join(REPO, "langevin_fts_amd", "csrc", "hip")
+    names = set()
+    for f in os.listdir(src):
+        names |= set(re.findall(r"^\s*#\s*(?:ifndef|ifdef)\s+(FTS_\w+)", open(os.path.join(src, f)).read(), flags=re.M))
+    assert names <= {"FTS_DYNAMIC_LDS"}

@@ -1094,6 +1094,7 @@ __global__ void __launch_bounds__(1024) line_steps_kernel(int n, FlatBatch<T> ba
     double* xa = half + n;                                // inputs of the three convolutions, two buffers each
     double* xb = xa + 2 * n;
     double* xc = xb + 2 * n;
+    double* parts = xc + 2 * n;                           // partial sums of the coefficients
     const FlatItem<T>& it = batch.it[blockIdx.x];
     const int nzc = n / 2 + 1;
     // P neighbouring lanes share point i; lane p takes the inputs j = p (mod P)
@@ -1126,17 +1127,59 @@ __global__ void __launch_bounds__(1024) line_steps_kernel(int n, FlatBatch<T> ba
         full[m] = sum / n;
     }
     __syncthreads();
-    if (threadIdx.x < (CONTINUOUS ? 2 : 1)) {
-        // the coefficients add up to b[0]: what rounding left of that would scale the field's mean
-        // in every step
-        double* c = threadIdx.x == 0 ? full : half;
-        double left = threadIdx.x == 0 ? xb[0] : xc[0], lost = 0.0;
-        for (int k = 0; k < n; k++) {
-            const double y = -c[k] - lost, next = left + y;
-            lost = (next - left) - y;
-            left = next;
+    // The coefficients add up to b[0]: what rounding left of that would scale the field's mean in every
+    // step (half an ulp of c[0] is 2^-54 a convolution: 1e-14 after 100 steps, 3 to 4 times the error of
+    // transforms at 16 and 64 points). The roots' errors, which leave much the same in every
+    // coefficient, go back evenly, where only the mean sees it; then c[0] takes the rest, and
+    // its neighbours in turn what the finer grid of their values holds of it, nearest first, where every
+    // mode of a smooth field weighs them alike.
+    constexpr int BONDS = CONTINUOUS ? 2 : 1;
+    const bool owner = threadIdx.x < BONDS;
+    double* c = threadIdx.x == 0 ? full : half;
+    // b[0] less the coefficients, every addition with its rounding error: LINE_PARTS partial sums, then the
+    // owner of a bond adds them (one thread's walk over 128 coefficients is 2 us of a launch)
+    auto rest = [&] {
+        if (threadIdx.x < BONDS * LINE_PARTS) {
+            const double* v = full + threadIdx.x / LINE_PARTS * n;
+            double s = 0.0, lost = 0.0;
+            for (int k = threadIdx.x % LINE_PARTS; k < n; k += LINE_PARTS) {
+                const double t = s + v[k], z = t - s;
+                lost += (s - (t - z)) + (v[k] - z);
+                s = t;
+            }
+            parts[2 * threadIdx.x] = s;
+            parts[2 * threadIdx.x + 1] = lost;
         }
-        c[0] += left;
+        __syncthreads();
+        double s = threadIdx.x == 0 ? xb[0] : xc[0], lost = 0.0;
+        if (owner)
+            for (int k = LINE_PARTS * threadIdx.x; k < LINE_PARTS * (threadIdx.x + 1); k++) {
+                const double x = -parts[2 * k], t = s + x, z = t - s;
+                lost += (s - (t - z)) + (x - z) - parts[2 * k + 1];
+                s = t;
+            }
+        return s + lost;
+    };
+    double left = rest();
+    if (owner) xa[threadIdx.x] = left / n;
+    __syncthreads();
+    for (int m = threadIdx.x; m < BONDS * n; m += blockDim.x) full[m] += xa[m < n ? 0 : 1];
+    __syncthreads();
+    left = rest();
+    if (owner) {
+        // 2^-61: 1e-16 of the mean after 300 convolutions
+        for (int d = 0; 2 * d <= n && fabs(left) > 0x1p-61; d++) {
+            const int e = d == 0 ? 0 : n - d;
+            const double share = e == d ? left : 0.5 * left;
+            const double a = c[d] + share;
+            left -= a - c[d];
+            c[d] = a;
+            if (e != d) {
+                const double b = c[e] + share;
+                left -= b - c[e];
+                c[e] = b;
+            }
+        }
     }
     __syncthreads();
     T* q = it.q;

@@ -216,6 +216,7 @@ struct FlatBatch {
 // share a point: at most 1024 threads
 constexpr int LINE_POINTS = 256;
 constexpr int line_lanes(int n) { return n <= 128 ? 8 : 4; }
-constexpr size_t line_lds(int n) { return sizeof(double) * 8 * (size_t)n; }
+constexpr int LINE_PARTS = 8;   // partial sums per bond of its coefficients
+constexpr size_t line_lds(int n) { return sizeof(double) * (8 * (size_t)n + 4 * LINE_PARTS); }
 
 }  // namespace fts

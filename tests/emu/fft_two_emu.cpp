@@ -16,6 +16,7 @@
 //    flat: the same two steps by flat_steps_kernel (nx = 1)
 //    flatd: two discrete steps by flat_steps_kernel (nx = 1)
 //    line, lined: the same by line_steps_kernel with one lane per point (nx = ny = 1)
+//    linec: the coefficients that line_steps_kernel makes of the full and the half bond (nx = ny = 1, FP64)
 // Bond factors along each axis: exp(-0.3 (k / L)^2) full, exp(-0.15 (k / L)^2) half, k folded.
 #include <hip/hip_runtime.h>
 
@@ -32,7 +33,7 @@
 namespace fts {
 unsigned char* smem_raw_ptr;
 }
-inline double cospi(double x) { return std::cos(M_PI * x); }
+inline double cospi(double x) { return (double)cosl(3.14159265358979323846264338327950288L * x); }
 inline double __shfl_xor(double v, int, int) { return v; }   // groups of one lane only
 #define FTS_DYNAMIC_LDS(name) unsigned char* name = smem_raw_ptr
 #include "fts_fft_two.hpp"
@@ -59,6 +60,7 @@ void* scheduler_fake = nullptr;
 const void* scheduler_stack = nullptr;
 size_t scheduler_size = 0;
 size_t current = 0;
+std::vector<float> lds_left;   // what the last workgroup left in its LDS
 void (*body)(void*) = nullptr;
 void* body_arg = nullptr;
 
@@ -127,6 +129,7 @@ void run_grid(dim3 grid, int threads, size_t lds, F&& kernel) {
                         std::exit(4);
                     }
             }
+            lds_left = mem;
         }
 }
 
@@ -288,13 +291,13 @@ int run(const char* op, const int* n, const char* in_path, const char* out_path)
             it.half = half.data();
             it.w = w.data();
             it.mask = mask.data();
-            it.steps = 2;
+            it.steps = is("linec") ? 0 : 2;
             it.full_table = 0;
             it.half_table = 1;
-            const bool cont = is("flat") || is("line");
+            const bool cont = is("flat") || is("line") || is("linec");
             it.full_w = cont ? half_w : full_w;
             it.half_w = quarter_w;
-            if (is("line") || is("lined")) {
+            if (is("line") || is("lined") || is("linec")) {
                 run_grid(dim3{1, 1, 1}, (n[2] + 63) / 64 * 64, fts::line_lds(n[2]), [&] {
                     if (cont) fts::line_steps_kernel<T, true, 1, 0>(n[2], b, e.bz.data());
                     else fts::line_steps_kernel<T, false, 1, 128>(n[2], b, e.bz.data());
@@ -307,6 +310,7 @@ int run(const char* op, const int* n, const char* in_path, const char* out_path)
                     fts::flat_steps_kernel<T, false>(e.g, b, e.tw[1].data(), e.tw[2].data(), e.by.data(), e.bz.data());
             });
             std::copy(q.begin() + M, q.end(), out.begin());
+            if (is("linec")) std::memcpy(out.data(), lds_left.data(), 2 * M * sizeof(T));
         }
     }
     FILE* f = std::fopen(out_path, "wb");

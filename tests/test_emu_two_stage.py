@@ -8,6 +8,7 @@ Nyquist column), more butterflies than threads, and the plans' limits. CPU only.
 
 Tolerances: a transform's rounding error grows as eps log2(M) in the 2-norm; 64 eps bounds each
 result's largest error over its largest value for the steps' 12 transforms at these sizes."""
+import fractions
 import os
 import shutil
 import subprocess
@@ -113,3 +114,20 @@ def test_two_stage_fp64(exe, n, tmp_path):
 def test_two_stage_fp32(exe, n, tmp_path):
     ops = ["fft", "ifft", "conv", "step"] + flat_ops(n)
     check(exe, n, 4, ops, str(tmp_path))
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 16, 30, 64, 105, 128, 256])
+def test_line_coefficients(exe, n, tmp_path):
+    """The coefficients of a line's direct convolutions act the same way in every step: each within an ulp or two of
+    the bond factors' inverse transform (longdouble), and their sum, which scales the field's mean, 1 to 2^-60 (the
+    rounding of the largest one alone would leave 2^-54, 1e-14 of the mean after 100 steps)."""
+    c = run(exe, "linec", 8, (1, 1, n), np.ones(3 * n), str(tmp_path)).reshape(2, n)
+    k = np.arange(n // 2 + 1)
+    for row, share in zip(c, (0.3, 0.15)):
+        b = np.exp(-share * k * k / n / n)
+        ref = np.fft.irfft(b.astype(np.longdouble), n) if n > 1 else b.astype(np.longdouble)
+        assert ref.dtype == np.longdouble
+        exact = sum((fractions.Fraction(float(x)) for x in row), fractions.Fraction(-1))
+        print(n, share, f"sum - 1 {float(exact):.1e}", f"coefficients {float(np.max(np.abs(row - ref))):.1e}")
+        assert abs(exact) < 2.0 ** -60
+        assert np.max(np.abs(row - ref)) < 2 * 2.0 ** -53

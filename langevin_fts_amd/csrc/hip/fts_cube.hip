@@ -16,6 +16,9 @@ void slab(const Grid& g, int mode, const SlabBatch<T>& b) {
     using T2 = typename vec2<T>::type;
     const dim3 grid(N, b.n), block(BD);
     const size_t lds = two_slab_lds(TwoCube<N, sizeof(T2)>::G, sizeof(T2));
+    for (int i = 0; i < b.n; i++)
+        if ((mode == SLAB_INV2 || (mode == SLAB_FWD && b.it[i].n_out > 1)) && !b.it[i].w)
+            throw Error("slab item of two spectra without a factor table");
     const T2 *twy = g.tw<T>(1), *twz = g.tw<T>(2);
     if (mode == SLAB_FWD)
         hipLaunchKernelGGL((slab_cube_kernel<T, SLAB_FWD, N, BD>), grid, block, lds, g.stream(), b, twy, twz);

@@ -18,6 +18,8 @@
 // with the Hermitian identities; this works for odd and even lengths alike.
 #pragma once
 
+#include <type_traits>
+
 #include "fts_common.hpp"
 
 namespace fts {
@@ -323,6 +325,7 @@ struct SlabItem {
     typename vec2<T>::type* c1;
     const T* w;        // factor table, see factor(); nullptr: all factors 1
     const T* mask;     // nullptr: no mask
+    // factor coefficients; with FP64 tables post1 and pre1 are FACTOR_ROOT, post0 and pre0 FACTOR_TABLE, or 0
     T post0, post1;    // inverse part: r_o *= factor(post_o) / M
     T pre0, pre1;      // forward part: spectrum_o = FFT[factor(pre_o) q]
     int n_out;         // FWD mode: 1 or 2 spectra
@@ -450,13 +453,54 @@ __device__ __forceinline__ void store_spectrum(const T2* S, const SlabGeom& g, T
     }
 }
 
+// Square root of a factor in FP64 to 0.5 ulp and a little: one Goldschmidt step from the hardware's
+// reciprocal root (about 2^-26) and one correction by the remainder, 8 operations where the library's
+// root, which scales small arguments, takes twice as many (5% of a 64^3 evaluation). Below 2^-767 the
+// remainder is rounded and a few ulp are lost. 0, infinity and NaN are their own roots.
+__device__ __forceinline__ double factor_root(double x) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const double y = __builtin_amdgcn_rsq(x);
+#else
+    const double y = 1.0 / sqrt(x);
+#endif
+    double g = x * y, h = 0.5 * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return x > 0.0 && x < __builtin_huge_val() ? g : x;
+}
+
 // The step factor of a point, from a table of exponentials made once per call: FACTOR_TABLE takes
-// the value as it is, FACTOR_SQUARE squared; coef 0 or no table: 1.
-constexpr double FACTOR_TABLE = -1.0, FACTOR_SQUARE = -2.0;
+// the value as it is; coef 0 or no table: 1. Continuous steps take two factors, one the square of
+// the other. FP64 tables hold the square, FACTOR_ROOT takes its root: a product of rounded values
+// would have twice their error and its own, the same way in every step. (A table for each cost 6% of
+// an evaluation at 48 x 84 x 60 and 30% at 60 x 104, the root 1.5% and nothing.) FP32 tables, rounded from FP64
+// exponentials, hold the root, FACTOR_SQUARE squares it.
+constexpr double FACTOR_TABLE = -1.0, FACTOR_SQUARE = -2.0, FACTOR_ROOT = -3.0;
 template <typename T>
 __device__ __forceinline__ T factor(T w, bool has_w, T coef) {
     if (!has_w || coef == (T)0) return (T)1;
-    return coef == (T)FACTOR_SQUARE ? w * w : w;
+    if constexpr (std::is_same<T, double>::value) return coef == FACTOR_ROOT ? factor_root(w) : w;
+    else return coef == (T)FACTOR_SQUARE ? w * w : w;
+}
+// The same for a kernel of constant geometry: ROOT, the factor of an item's second spectrum (post1, pre1),
+// which always has a table. The root is made at each use, from a value that is opaque to the compiler, and under
+// no condition: else it makes the roots of all of a thread's points before the first use, or keeps
+// them from the inverse to the forward transform (132 against 108 registers at 48^3, which take a
+// wavefront of every SIMD, 212 against 184 at 64^3).
+template <bool ROOT, typename T>
+__device__ __forceinline__ T factor_at(T w, bool has_w, T coef) {
+    if constexpr (ROOT && std::is_same<T, double>::value) {
+#ifdef __HIP_DEVICE_COMPILE__
+        asm volatile("" : "+v"(w));
+#endif
+        return factor_root(w);
+    } else if constexpr (std::is_same<T, double>::value) {
+        return has_w && coef != (T)0 ? w : (T)1;
+    } else {
+        return factor<T>(w, has_w, coef);
+    }
 }
 
 // write this thread's real values times exp(-w*coef) into the packed rows

@@ -685,6 +685,7 @@ __global__ void __launch_bounds__(BD) slab_cube_kernel(SlabBatch<T> batch, const
     // a fetched spectrum -> real values times factor(coef) / M; COMB: (4 x - q) / 3 against the
     // values already in q. `between`: loads to issue once the spectrum has left its registers.
     auto inverse = [&](T2 (&v)[YT][RY], T coef, auto comb, auto&& between) {
+        constexpr bool COMB = decltype(comb)::value;
 #pragma unroll
         for (int k = 0; k < YT; k++) {
             int c, j;
@@ -710,16 +711,17 @@ __global__ void __launch_bounds__(BD) slab_cube_kernel(SlabBatch<T> batch, const
                 RDft<RZ, +1, T, T2>::run(u);
 #pragma unroll
                 for (int r = 0; r < RZ; r++) {
-                    const T xe = u[r].x * factor<T>(we[k][r], has_w, coef) * inv_m;
-                    const T xo = u[r].y * factor<T>(wo[k][r], has_w, coef) * inv_m;
-                    qe[k][r] = decltype(comb)::value ? ((T)4.0 * xe - qe[k][r]) / (T)3.0 : xe;
-                    qo[k][r] = decltype(comb)::value ? ((T)4.0 * xo - qo[k][r]) / (T)3.0 : xo;
+                    const T xe = u[r].x * factor_at<COMB>(we[k][r], has_w, coef) * inv_m;
+                    const T xo = u[r].y * factor_at<COMB>(wo[k][r], has_w, coef) * inv_m;
+                    qe[k][r] = COMB ? ((T)4.0 * xe - qe[k][r]) / (T)3.0 : xe;
+                    qo[k][r] = COMB ? ((T)4.0 * xo - qo[k][r]) / (T)3.0 : xo;
                 }
             }
         }
     };
     // real values times factor(coef) -> spectrum
-    auto forward = [&](T coef, T2* spec) {
+    auto forward = [&](T coef, auto root, T2* spec) {
+        constexpr bool ROOT = decltype(root)::value;
 #pragma unroll
         for (int k = 0; k < ZT; k++) {
             int j, i0;
@@ -728,8 +730,8 @@ __global__ void __launch_bounds__(BD) slab_cube_kernel(SlabBatch<T> batch, const
                 T2 u[RZ];
 #pragma unroll
                 for (int r = 0; r < RZ; r++)
-                    u[r] = T2{qe[k][r] * factor<T>(we[k][r], has_w, coef) * (T)0.5,
-                              qo[k][r] * factor<T>(wo[k][r], has_w, coef) * (T)0.5};
+                    u[r] = T2{qe[k][r] * factor_at<ROOT>(we[k][r], has_w, coef) * (T)0.5,
+                              qo[k][r] * factor_at<ROOT>(wo[k][r], has_w, coef) * (T)0.5};
                 RDft<RZ, -1, T, T2>::run(u);
 #pragma unroll
                 for (int r = 1; r < RZ; r++) u[r] = tmul(u[r], z_root(r, j));
@@ -799,10 +801,10 @@ __global__ void __launch_bounds__(BD) slab_cube_kernel(SlabBatch<T> batch, const
         }
         if (!it.forward) return;
     }
-    forward(it.pre0, it.c0 + coff);
+    forward(it.pre0, std::false_type{}, it.c0 + coff);
     if (n_out < 2) return;
     __syncthreads();   // the plane of the first spectrum is read
-    forward(it.pre1, it.c1 + coff);
+    forward(it.pre1, std::true_type{}, it.c1 + coff);
 }
 
 // ------------------------------------------------------------------ pencil (x) pass
@@ -1183,9 +1185,10 @@ __global__ void __launch_bounds__(1024) line_steps_kernel(int n, FlatBatch<T> ba
     }
     __syncthreads();
     T* q = it.q;
-    const double f = on ? (double)it.w[i] : 0.0;
-    // discrete: exp(-w ds); continuous: exp(-w ds/4) and its square, rounded as the slab passes' are
-    const double e4 = f, e2 = CONTINUOUS ? (double)((T)f * (T)f) : 0.0;
+    // discrete: exp(-w ds), in e2; continuous: exp(-w ds/2) and exp(-w ds/4), as the slab passes take them
+    const T f = on ? it.w[i] : (T)0;
+    const double e2 = (double)factor<T>(f, true, it.full_w);
+    const double e4 = CONTINUOUS ? (double)factor<T>(f, true, it.half_w) : 0.0;
     const double mask = on && it.mask ? (double)it.mask[i] : 1.0;
     double x = on ? (double)q[i] : 0.0;
     // this lane's coefficients c[(i - j) mod n] of j = p + P t, and the places of v[j]: in registers
@@ -1233,7 +1236,7 @@ __global__ void __launch_bounds__(1024) line_steps_kernel(int n, FlatBatch<T> ba
             __syncthreads();
             x = (4.0 * (e4 * conv(ch, half, c)) - q1) / 3.0 * mask;
         } else {
-            x = e4 * conv(cf, full, a) * mask;
+            x = e2 * conv(cf, full, a) * mask;
         }
         x = (double)(T)x;   // the stored slice is what the next step starts from
         q += batch.stride;

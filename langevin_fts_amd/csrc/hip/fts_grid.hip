@@ -481,7 +481,8 @@ TuneChoice tune_wave_local(const Grid& g) {
     // among the candidates, timed alone (the pencil pass does not depend on it)
     SlabBatch<T> sc = sb;
     for (int i = 0; i < ITEMS; i++) {
-        sc.it[i].post0 = sc.it[i].pre0 = (T)FACTOR_SQUARE;
+        if (std::is_same<T, double>::value) sc.it[i].post1 = sc.it[i].pre1 = (T)FACTOR_ROOT;
+        else sc.it[i].post0 = sc.it[i].pre0 = (T)FACTOR_SQUARE;
         sc.it[i].n_out = 2;
     }
     for (int mode : {SLAB_FWD, SLAB_INV2}) {

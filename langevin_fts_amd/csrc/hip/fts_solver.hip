@@ -91,15 +91,16 @@ private:
     T* slice_ptr(int p, int n, int half) const { return half ? h(p, n) : q(p, n); }
     const T* w(int m) const { return wT_ + (size_t)m * M_; }
     // the steps' exponential of monomer m, made once per compute_propagators from FP64 exponentials:
-    // exp(-w ds) of discrete chains, exp(-w ds/4) of continuous ones, whose exp(-w ds/2) is its square,
-    // exp(-w ds/2) of real-space steps
+    // exp(-w ds) of discrete chains, exp(-w ds/2) of real-space steps, exp(-w ds/2) (FP64) or exp(-w ds/4)
+    // (FP32) of continuous ones, from which the kernels take the other by a root or a square
     // (a Richardson step evaluated five exponentials per point, 10% of a 64^3 FP64 evaluation; in
     // FP32 the time is the same, and the rounded FP64 value has none of the hardware exponential's bias)
-    double table_arg() const { return model_ == FTS_DISCRETE ? ds_ : real_ ? ds_ / 2 : ds_ / 4; }
+    static constexpr bool FP64 = std::is_same<T, double>::value;
+    double table_arg() const { return model_ == FTS_DISCRETE ? ds_ : FP64 ? ds_ / 2 : ds_ / 4; }
     const T* ew(int m) const { return ew_.as<T>() + (size_t)m * M_; }
-    T ew_full() const { return (T)FACTOR_TABLE; }        // discrete: exp(-w ds)
-    T ew_half() const { return (T)FACTOR_SQUARE; }       // continuous: exp(-w ds/2)
-    T ew_quarter() const { return (T)FACTOR_TABLE; }     // continuous: exp(-w ds/4)
+    T ew_full() const { return (T)FACTOR_TABLE; }                               // discrete: exp(-w ds)
+    T ew_half() const { return (T)(FP64 ? FACTOR_TABLE : FACTOR_SQUARE); }      // continuous: exp(-w ds/2)
+    T ew_quarter() const { return (T)(FP64 ? FACTOR_ROOT : FACTOR_TABLE); }     // continuous: exp(-w ds/4)
     T2* slot(int s) const { return ws_.as<T2>() + (size_t)s * Ms_; }
     const T* mask() const { return g_->mask_h.empty() ? nullptr : g_->mask<T>(); }
     int full(int m) const { return 2 * m; }

@@ -16,6 +16,7 @@
 //    flat: the same two steps by flat_steps_kernel (nx = 1)
 //    flatd: two discrete steps by flat_steps_kernel (nx = 1)
 //    line, lined: the same by line_steps_kernel with one lane per point (nx = ny = 1)
+//    factor: exp(-w ds/2) and exp(-w ds/4) as the steps take them, w in the place of q
 //    linec: the coefficients that line_steps_kernel makes of the full and the half bond (nx = ny = 1, FP64)
 // Bond factors along each axis: exp(-0.3 (k / L)^2) full, exp(-0.15 (k / L)^2) half, k folded.
 #include <hip/hip_runtime.h>
@@ -242,12 +243,19 @@ int run(const char* op, const int* n, const char* in_path, const char* out_path)
     } else {
         // input: q, w, mask
         std::vector<T> w(in.begin() + M, in.begin() + 2 * M), mask(in.begin() + 2 * M, in.begin() + 3 * M);
-        // factors are read from a table: exp(-w ds/4) or, of discrete steps, exp(-w ds)
+        // factors are read from a table: exp(-w ds) of discrete steps, else exp(-w ds/2) in FP64 and exp(-w ds/4)
         const double ds = 0.25;
-        for (T& x : w) x = (T)std::exp(-(double)x * (is("flatd") || is("lined") ? ds : ds / 4));
-        const T half_w = (T)fts::FACTOR_SQUARE, quarter_w = (T)fts::FACTOR_TABLE, full_w = (T)fts::FACTOR_TABLE;
+        constexpr bool fp64 = sizeof(T) == 8;
+        for (T& x : w) x = (T)std::exp(-(double)x * (is("flatd") || is("lined") ? ds : fp64 ? ds / 2 : ds / 4));
+        const T half_w = (T)(fp64 ? fts::FACTOR_TABLE : fts::FACTOR_SQUARE), full_w = (T)fts::FACTOR_TABLE;
+        const T quarter_w = (T)(fp64 ? fts::FACTOR_ROOT : fts::FACTOR_TABLE);
         out.assign(2 * M, (T)NAN);
-        if (is("step")) {
+        if (is("factor")) {
+            for (size_t i = 0; i < M; i++) {
+                out[i] = fts::factor<T>(w[i], true, half_w);
+                out[M + i] = fts::factor<T>(w[i], true, quarter_w);
+            }
+        } else if (is("step")) {
             std::vector<T> q(in.begin(), in.begin() + M);
             auto c0 = e.spectrum(), c1 = e.spectrum();
             fts::SlabItem<T> a{};

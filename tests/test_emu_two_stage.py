@@ -131,3 +131,32 @@ def test_line_coefficients(exe, n, tmp_path):
         print(n, share, f"sum - 1 {float(exact):.1e}", f"coefficients {float(np.max(np.abs(row - ref))):.1e}")
         assert abs(exact) < 2.0 ** -60
         assert np.max(np.abs(row - ref)) < 2 * 2.0 ** -53
+
+
+@pytest.mark.parametrize("esize,bars", [(8, (0.53, 0.88)), (4, (1.92, 0.53))])
+def test_step_factors(exe, esize, bars, tmp_path):
+    """The factors exp(-w ds/2) and exp(-w ds/4) of a continuous step against longdouble. FP64: a rounded value (0.5 ulp,
+    and the exponential's own 0.02) and its rounded root (half of that relative error, at most sqrt(2) / 4 ulp of the
+    root, and 0.5 more). FP32: a product of two rounded values (twice the error, at most sqrt(2) ulp of the product,
+    and 0.5 more) and a rounded value."""
+    n = (1, 1, 256)
+    w = np.random.default_rng(8).uniform(-40, 40, 256)
+    if esize == 4:
+        w = w.astype(np.float32).astype(np.float64)
+    got = run(exe, "factor", esize, n, np.concatenate([w, w, w]), str(tmp_path)).reshape(2, -1)
+    for row, coef, bar in zip(got, (0.125, 0.0625), bars):
+        ref = np.exp(-w.astype(np.longdouble) * coef)
+        ulp = np.spacing(ref.astype(np.float32 if esize == 4 else np.float64)).astype(np.longdouble)
+        e = float(np.max(np.abs(row - ref) / ulp))
+        print(esize, coef, f"{e:.2f} ulp")
+        assert e < bar
+
+
+def test_step_factors_at_their_limits(exe, tmp_path):
+    """Factors of walls and wells: 0, infinity and NaN pass, tiny and huge ones keep their precision (FP64)."""
+    w = np.array([np.inf, -np.inf, np.nan, 4000.0, -4000.0, 1e300, -1e300, 0.0])
+    got = run(exe, "factor", 8, (1, 1, 8), np.concatenate([w, w, w]), str(tmp_path)).reshape(2, -1)
+    for row, coef in zip(got, (0.125, 0.0625)):
+        with np.errstate(over="ignore"):
+            ref = np.exp(-w * coef)
+        assert np.allclose(row, ref, rtol=1e-13, atol=0.0, equal_nan=True), (row, ref)

@@ -15,7 +15,7 @@
 //          forward, INV2 with forward), twice; input: q, w, mask; output: both slices
 //    flat: the same two steps by flat_steps_kernel (nx = 1)
 //    flatd: two discrete steps by flat_steps_kernel (nx = 1)
-//    line, lined: the same by line_steps_kernel with one lane per point (nx = ny = 1)
+//    line, lined: the same by line_steps_kernel in the launch shape of the length (nx = ny = 1)
 //    factor: exp(-w ds/2) and exp(-w ds/4) as the steps take them, w in the place of q
 //    linec: the coefficients that line_steps_kernel makes of the full and the half bond (nx = ny = 1, FP64)
 // Bond factors along each axis: exp(-0.3 (k / L)^2) full, exp(-0.15 (k / L)^2) half, k folded.
@@ -35,7 +35,7 @@ namespace fts {
 unsigned char* smem_raw_ptr;
 }
 inline double cospi(double x) { return (double)cosl(3.14159265358979323846264338327950288L * x); }
-inline double __shfl_xor(double v, int, int) { return v; }   // groups of one lane only
+double __shfl_xor(double v, int mask, int width);
 #define FTS_DYNAMIC_LDS(name) unsigned char* name = smem_raw_ptr
 #include "fts_fft_two.hpp"
 
@@ -84,6 +84,16 @@ void fiber_main() {
 void emu_syncthreads() {
     fibers[current].barriers++;
     to_scheduler(false);
+}
+
+// every thread of the workgroup takes part, as in the kernels: one round of the ring stores, the next one reads
+double __shfl_xor(double v, int mask, int) {
+    static double lanes[1024];
+    lanes[current] = v;
+    emu_syncthreads();
+    const double r = lanes[current ^ (size_t)mask];
+    emu_syncthreads();
+    return r;
 }
 
 namespace {
@@ -306,9 +316,17 @@ int run(const char* op, const int* n, const char* in_path, const char* out_path)
             it.full_w = cont ? half_w : full_w;
             it.half_w = quarter_w;
             if (is("line") || is("lined") || is("linec")) {
-                run_grid(dim3{1, 1, 1}, (n[2] + 63) / 64 * 64, fts::line_lds(n[2]), [&] {
-                    if (cont) fts::line_steps_kernel<T, true, 1, 0>(n[2], b, e.bz.data());
-                    else fts::line_steps_kernel<T, false, 1, 128>(n[2], b, e.bz.data());
+                const int L = n[2], P = fts::line_lanes(L);
+                run_grid(dim3{1, 1, 1}, (L * P + 63) / 64 * 64, fts::line_lds(L), [&] {
+                    auto go = [&](auto p, auto ch) {
+                        constexpr int PP = decltype(p)::value, CH = decltype(ch)::value;
+                        if (cont) fts::line_steps_kernel<T, true, PP, CH>(L, b, e.bz.data());
+                        else fts::line_steps_kernel<T, false, PP, CH>(L, b, e.bz.data());
+                    };
+                    using std::integral_constant;
+                    if (L <= 64) go(integral_constant<int, 8>{}, integral_constant<int, 8>{});
+                    else if (L <= 128) go(integral_constant<int, 8>{}, integral_constant<int, 16>{});
+                    else go(integral_constant<int, 4>{}, integral_constant<int, 0>{});
                 });
             } else
             run_grid(dim3{1, 1, 1}, fts::two_slab_threads(e.g), fts::two_slab_lds(e.g, sizeof(T2)), [&] {

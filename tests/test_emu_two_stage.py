@@ -3,8 +3,9 @@ tests/emu/fft_two_emu.cpp and run as emulated workgroups with AddressSanitizer o
 and on every global buffer (NaN in what was never written): forward and inverse transforms
 against numpy, a convolution with the bond factors, and two masked propagator steps of each kind
 by the slab and pencil passes and by the one-launch kernels of flat grids, against numpy in FP64.
-The grids take every radix 1..16 on the axes, odd and even lengths (rows without a partner, no
-Nyquist column), more butterflies than threads, and the plans' limits. CPU only.
+The grids take every radix 1..16 as r1 or r2 of each axis, odd and even lengths (rows without a
+partner, no Nyquist column), more butterflies than threads, the longest axis and planes that fill the
+LDS. CPU only.
 
 Tolerances: a transform's rounding error grows as eps log2(M) in the 2-norm; 64 eps bounds each
 result's largest error over its largest value for the steps' 12 transforms at these sizes."""
@@ -98,10 +99,44 @@ def flat_ops(n):
     return (["flat", "flatd"] if n[0] == 1 else []) + (["line", "lined"] if n[0] == n[1] == 1 else [])
 
 
-# (x, y, z): every radix as r1 and as r2 of a y and of a z plan, odd and even lengths
+# (x, y, z): odd and even lengths of every radix; test_grids_take_every_radix
 GRIDS = [(2, 8, 8), (3, 6, 10), (4, 12, 9), (5, 15, 16), (7, 14, 26), (11, 22, 33), (13, 21, 35), (2, 45, 20),
          (6, 7, 13), (1, 60, 104), (1, 1, 128), (1, 1, 30), (2, 30, 27), (9, 10, 1), (16, 3, 4), (2, 49, 25),
-         (1, 9, 11), (3, 1, 24)]
+         (1, 9, 11), (3, 1, 24), (208, 3, 2), (225, 2, 2), (196, 1, 3), (144, 2, 5), (2, 169, 6), (1, 225, 8),
+         (1, 240, 4), (2, 182, 5), (1, 256, 6), (1, 144, 10), (1, 6, 196), (1, 4, 225), (1, 3, 240), (1, 2, 256),
+         (1, 5, 144), (1, 2, 182), (60, 1, 2), (72, 1, 2)]
+# planes of 140 KB and more of LDS
+PLANES = [(1, 126, 126), (1, 84, 182), (1, 112, 128)]
+GRIDS32 = [(2, 8, 8), (3, 6, 10), (5, 15, 16), (1, 20, 48), (1, 1, 128), (225, 2, 2), (240, 2, 2), (144, 1, 3),
+           (100, 2, 3), (72, 1, 2), (1, 225, 4), (1, 256, 3), (2, 150, 5), (1, 144, 4), (1, 72, 8), (1, 3, 225),
+           (1, 2, 256), (1, 4, 144), (1, 2, 64), (1, 100, 150), (1, 1, 72), (1, 1, 256), (1, 3, 9), (24, 1, 2),
+           (1, 36, 2)]
+LINES = [(1, 1, 2), (1, 1, 63), (1, 1, 64), (1, 1, 65), (1, 1, 130), (1, 1, 225), (1, 1, 256)]
+
+
+def two_axis(L, y, fp32):
+    """fts_two_plan.hpp's rule: the smallest larger radix; on y the first radix is even, or the larger one of an odd
+    length; FP32 has no 7, 11 or 13"""
+    ok = [r for r in range(1, 17) if not (fp32 and any(r % p == 0 for p in (7, 11, 13)))]
+    m, s = next((m, s) for m in ok for s in ok if s <= m and m * s == L)
+    return (m, s) if y and (L % 2 == 1 or s % 2 == 1) else (s, m)
+
+
+def test_grids_take_every_radix():
+    for axis in range(3):
+        for fp32, grids in ((False, GRIDS + PLANES + LINES), (True, GRIDS32)):
+            seen = {r for n in grids for r in two_axis(n[axis], axis == 1, fp32)}
+            assert seen >= {r for r in range(1, 17) if not fp32 or r % 7 and r % 11 and r % 13}, (axis, fp32, seen)
+
+
+@pytest.mark.parametrize("n", LINES)
+def test_lines_fp64(exe, n, tmp_path):
+    check(exe, n, 8, ["line", "lined"], str(tmp_path))
+
+
+@pytest.mark.parametrize("n", PLANES)
+def test_full_planes_fp64(exe, n, tmp_path):
+    check(exe, n, 8, ["conv", "flat"], str(tmp_path))
 
 
 @pytest.mark.parametrize("n", GRIDS)
@@ -110,7 +145,7 @@ def test_two_stage_fp64(exe, n, tmp_path):
     check(exe, n, 8, ops, str(tmp_path))
 
 
-@pytest.mark.parametrize("n", [(2, 8, 8), (3, 6, 10), (5, 15, 16), (1, 20, 48), (1, 1, 128)])
+@pytest.mark.parametrize("n", GRIDS32)
 def test_two_stage_fp32(exe, n, tmp_path):
     ops = ["fft", "ifft", "conv", "step"] + flat_ops(n)
     check(exe, n, 4, ops, str(tmp_path))

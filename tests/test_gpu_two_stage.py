@@ -88,6 +88,46 @@ def test_fp32(ctx, capi, nx):
     check(ctx, capi, "diblock_f0.5_ds1_90", "discrete", nx, "fp32")
 
 
+# FP32: a segment's factors are 2^-24 off or so at every point, in every step: 2e-5 is 300 segments' worth where all
+# act the same way, so chains of 100 segments keep it (the branched one has 276, with masks Q is 4e-6 and 2.04e-5 off)
+MODELS32 = [("diblock_f0.36_ds0.01", "continuous"), ("diblock_f0.5_ds1_90", "discrete")]
+
+
+@pytest.mark.parametrize("name,model", MODELS32)
+@pytest.mark.parametrize("nx", [[2], [64], [72], [128], [135], [256], [20, 48], [60, 64], [100, 150]])
+def test_fp32_lines_and_flat_grids(ctx, capi, nx, name, model):
+    """FP32 instances of the one-launch kernels, at the lengths where the line kernel's lanes and chunks change."""
+    say(f"fp32 one launch {nx} {model}")
+    check(ctx, capi, name, model, nx, "fp32")
+    rng = np.random.default_rng(4)
+    check(ctx, capi, name, model, nx, "fp32", mask=(rng.random(int(np.prod(nx))) > 0.1).astype(np.float64), stress=False)
+
+
+@pytest.mark.parametrize("nx", [[48] * 3, [64] * 3, [40, 45, 36]])
+def test_fp32_keeps_the_mean(ctx, capi, nx):
+    """The field's mean is not rounded to an FP32 sum of all points in every convolution: 100 continuous steps round that 300
+    times, 1e-6 on Q (measured rms of these fields with the mean in the x transform: 1.1e-6, 1.0e-6, 1.1e-6). Past
+    the x transform it keeps the planes' rounding: some 12 additions of 2^-24 / sqrt(12) each way, 6e-8 of a plane's mean,
+    over sqrt(nx) planes and sqrt(2 x 300) passes: 1.8e-7 at nx = 64. The bar on the rms of 6 fields is 2.5 times that;
+    the value is the FP64 solver's Q."""
+    plan = golden("plans")["diblock_f0.36_ds0.01|continuous|0"]
+    inp = plan["input"]
+    M = int(np.prod(nx))
+    g = capi.Grid(ctx, nx, [0.07 * n for n in nx])
+    P = capi.Plan(plan, inp["ds"], inp["bonds"], plan["schedules"]["4"])
+    s64, s32 = capi.Solver(g, P, capi.FTS_FP64), capi.Solver(g, P, capi.FTS_FP32)
+    err = []
+    for seed in range(6):
+        rng = np.random.default_rng(seed)
+        w = {m: 2.0 * rng.standard_normal(M).astype(np.float32).astype(np.float64) for m in inp["bonds"]}
+        s64.compute_propagators(w)
+        s32.compute_propagators(w)
+        err.append(s32.get_total_partition(0) / s64.get_total_partition(0) - 1)
+    rms = float(np.sqrt(np.mean(np.square(err))))
+    say(f"fp32 mean {nx}: Q errors {' '.join('%+.1e' % e for e in err)}, rms {rms:.1e}")
+    assert rms < 2.5 * 1.8e-7 * np.sqrt(64 / nx[0])
+
+
 @pytest.mark.parametrize("n", [15, 16, 17, 512, 1023, 1024, 1025])
 def test_realspace_lines(ctx, capi, n):
     say(f"real-space sweeps {n}")

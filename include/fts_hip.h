@@ -101,9 +101,12 @@ int fts_grid_fft_backward_noalloc(fts_grid* g, int precision, const void* d_in, 
  * precision, the grid picks the slab-pass workgroup size (slab_threads) and the kz
  * columns per wavefront of the pencil pass (pencil_columns) by timing the candidates
  * when it is created. Results of the candidates are bit-identical at 32^3 and 64^3,
- * where tuning is on by default; at 48^3, 96^3 and 128^3 they agree to rounding only,
- * so the defaults stay there unless the environment sets FTS_FFT_TUNE=1 (a timed
- * choice could differ between processes and with it a chaotic run's trajectory).
+ * where tuning is on by default; at 48^3, 96^3 and 128^3 they are promised to agree to
+ * rounding only (FP32 differs at 48^3 and 96^3 between some pencil widths), so the
+ * defaults stay there unless the environment sets FTS_FFT_TUNE=1 (a timed choice could
+ * differ between processes and with it a chaotic run's trajectory). Launches of more
+ * than four propagators at 64^3 take workgroups of their own, whatever was tuned, until
+ * set is called.
  * FTS_FFT_TUNE=0 keeps the defaults everywhere. The default pencil_columns is 8, and
  * 4 in FP64 from 96^3. One process keeps one choice per (N, precision). slab_threads is
  * the half step's (discrete

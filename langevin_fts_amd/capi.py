@@ -242,7 +242,8 @@ class Grid:
 
     def fft_schedule(self, precision=FTS_FP64):
         """(slab workgroup threads, pencil kz columns per wavefront, note) of the
-        wave-local FFT kernels; (0, 0, ...) on grids without them."""
+        N^3 FFT kernels; (0, 0, ...) on grids without them. Launches of more than four
+        propagators at 64^3 take a shape of their own unless set_fft_schedule was called."""
         bd, nl = ctypes.c_int(), ctypes.c_int()
         buf = ctypes.create_string_buffer(512)
         check(lib().fts_grid_get_fft_schedule(self.h, precision, ctypes.byref(bd), ctypes.byref(nl), buf, 512))

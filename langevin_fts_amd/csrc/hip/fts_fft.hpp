@@ -475,7 +475,7 @@ __device__ __forceinline__ double factor_root(double x) {
 // the value as it is; coef 0 or no table: 1. Continuous steps take two factors, one the square of
 // the other. FP64 tables hold the square, FACTOR_ROOT takes its root: a product of rounded values
 // would have twice their error and its own, the same way in every step. (A table for each cost 6% of
-// an evaluation at 48 x 84 x 60 and 30% at 60 x 104, the root 1.5% and nothing.) FP32 tables, rounded from FP64
+// an evaluation at 48 x 84 x 60 and 30% at 60 x 104, the root 2 to 3% and nothing.) FP32 tables, rounded from FP64
 // exponentials, hold the root, FACTOR_SQUARE squares it.
 constexpr double FACTOR_TABLE = -1.0, FACTOR_SQUARE = -2.0, FACTOR_ROOT = -3.0;
 template <typename T>

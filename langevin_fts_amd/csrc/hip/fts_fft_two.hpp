@@ -74,9 +74,10 @@ __host__ __device__ constexpr double root_sin(int R, int m) {
     return R == 9 ? s9[m] : s16[m];
 }
 
-// Products are written as fused operations: the compiler's own choice of which product of a sum
-// to fuse can differ between instances of one kernel, and every launch shape of a grid gives the
-// same results.
+// Products with roots are written as fused operations: the compiler's own choice of which product of a sum
+// to fuse can differ between instances of one kernel. Lines of 32, 64 and 128 points so give the same bits in
+// every launch shape. Radices 3 and 5 and the prime ones leave their sums to the compiler: at 48^3 and 96^3
+// FP64 has been the same in all shapes, FP32 differs by 5e-7 between some pencil widths.
 __device__ __forceinline__ double two_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
 __device__ __forceinline__ float two_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 template <typename T2>
@@ -379,9 +380,9 @@ struct TwoPlane {
             });
         }
     }
-    // Stage A of z both ways around the real values: op(i0, two, v, vb) gets the index of a value
-    // of the pair's first row, whether the second row exists (at i0 + second), and the two
-    // values; it returns through them what the forward transform takes.
+    // Stage A of z both ways around the real values: op(i, two, v) gets the index of a value of the
+    // pair's first row, whether the second row exists (at i + second), and both values in v.x and
+    // v.y; it returns through them what the forward transform takes.
     template <typename Op>
     __device__ __forceinline__ void z_inner(bool inverse, bool forward, Op&& op) const {
         const int total = g.lines * g.zr2;
@@ -591,7 +592,10 @@ struct CubeSlab {
     // reads per transform pair. The shapes of few workgroups do: 64^3 with 320 threads 9.3 -> 8.9 and
     // 15.8 -> 15.2 us (half step, Richardson step of two propagators in FP64), 32^3 5.1 -> 4.8. In the
     // shapes of large batches the registers cost workgroups per CU (64^3 with 512 threads, 16
-    // propagators: 27 -> 37 us; the Richardson step of 32 propagators at 32^3: 14.6 -> 18.1 us).
+    // propagators: 27 -> 37 us; the Richardson step of 32 propagators at 32^3: 14.6 -> 18.1 us). 48^3 with
+    // 256 threads, its only default, has one butterfly per thread too and keeps the tables: in registers,
+    // evaluations of 2 propagators took 0.97 to 0.99 of the time in FP64, of 16 discrete ones 1.04, in FP32 1.05
+    // to 1.09 with 16.
     static constexpr bool ROOTS =
         (sizeof(T) == 8 && N == 64 && BD == 320) || (N == 32 && BD == 256 && MODE != SLAB_INV2);
     static_assert(!ROOTS || (ZT == 1 && G::nzc * G::y.r2 <= BD), "one butterfly per thread");
@@ -1086,7 +1090,7 @@ __global__ void __launch_bounds__(TWO_BD) flat_steps_kernel(TwoGeom geom, FlatBa
 // value in LDS or registers. Two barriers per Richardson step (a buffer is written again only two
 // barriers after its readers), where two butterflies each way and
 // the row pairing (with an empty partner) take eighteen: a step of 128 points took 23 us by
-// flat_steps_kernel, bound by those phases' latency, and takes 0.9 us. Sums are FP64 in either
+// flat_steps_kernel, bound by those phases' latency, and takes 2.2 us (50 steps of two propagators: 110 us). Sums are FP64 in either
 // precision.
 template <typename T, bool CONTINUOUS, int P, int CH>
 __global__ void __launch_bounds__(1024) line_steps_kernel(int n, FlatBatch<T> batch, const T* bz) {

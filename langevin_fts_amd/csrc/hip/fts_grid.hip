@@ -348,9 +348,10 @@ void Grid::setup_fft() {
     if (ct_n == 0) {
         // Every other grid takes the two-stage kernels when its lengths have such a plan and a plane
         // fits the LDS: a whole evaluation with them against the runtime-radix kernels of fts_fft.hpp
-        // (which keep lengths like 125, 17 k or above 256) measured 9.1 against 38.0 ms at 48x84x60
-        // (radix 7: those kernels run it from LDS twiddles and spill), 2.19 against 4.40 ms at
-        // 72x120x75 in FP32, 6.5 against 30.0 ms at 60x104 and 3.0 against 5.0 ms at 128 points in 1D.
+        // (which keep lengths like 125, 17 k or above 256) measures 7.9 against 38.0 ms at 48x84x60
+        // (radix 7: those kernels run it from LDS twiddles and spill) and 2.02 against 4.40 ms at
+        // 72x120x75 in FP32. Grids of one x-slab run their steps in one launch: 5.2 against 30.0 ms at
+        // 60x104, 0.52 against 5.0 ms at 128 points in 1D.
         // FP32 kernels carry no radix with a prime factor above 5, and big grids are refused in FP32
         two_stage[0] = two_geometry(tnx, sizeof(double2), LDS_LIMIT, two[0]);
         two_stage[1] = !big && two_geometry(tnx, sizeof(float2), LDS_LIMIT, two[1]);
@@ -373,7 +374,7 @@ void Grid::setup_fft() {
 // at least 2% faster.
 // The choice is cached per (N, precision) for the process. FTS_FFT_TUNE=0 keeps the
 // defaults. Candidates run the same per-line transforms; results agree to rounding
-// (bit-identical at 32^3 and 64^3, where the compiler contracts both alike).
+// (bit-identical at 32^3 and 64^3, whose radices leave the compiler no choice).
 namespace {
 struct TuneChoice {
     int bd, nl;
@@ -517,8 +518,9 @@ void Grid::tune_fft_schedule() {
     pencil_nl[p] = pencil_default_nl(ct_n, (int)sizeof(typename vec2<T>::type));
     // Tuning picks launch shapes by wall-clock timing, so the choice can differ between
     // processes. At 32^3 and 64^3 every candidate gives bit-identical results; at 48^3,
-    // 96^3 and 128^3 they differ by rounding, and a run could then follow another
-    // trajectory in another process: there the defaults stay unless FTS_FFT_TUNE=1.
+    // 96^3 and 128^3 they may differ by rounding (FP32 does at 48^3 and 96^3), and a run
+    // could then follow another trajectory in another process: there the defaults stay
+    // unless FTS_FFT_TUNE=1.
     const char* env = std::getenv("FTS_FFT_TUNE");
     const bool identical = ct_n == 32 || ct_n == 64;
     if (!wave_local || (env && env[0] == '0')) {

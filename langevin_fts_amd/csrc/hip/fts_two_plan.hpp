@@ -24,7 +24,8 @@ struct TwoAxis {
 // L = r1 r2 with the smallest larger radix. y axis: r1 even when L is (rows pair up inside a
 // butterfly), and the larger one when L is odd (one row of r1 has no partner). Other axes: the
 // larger radix is r2, the run of consecutive z values that a wavefront loads and stores; FP32
-// takes 4 x 16 for 64, runs of 64 bytes.
+// takes 4 x 16 for 64, runs of 64 bytes: evaluations with 8 x 8 took 1.05 to 1.09 of the time at
+// 40 x 48 x 64 and 72 x 60 x 64, 1.15 to 1.25 at 60 x 64, and 0.97 to 1.00 at 64^3.
 enum TwoAxisKind { TWO_X, TWO_Y, TWO_Z };
 constexpr bool two_axis(int L, TwoAxisKind kind, bool fp32, TwoAxis& a) {
     a = TwoAxis{L, 0, 0};
@@ -186,7 +187,9 @@ constexpr int slab_default_bd_mode(int N, int elem_bytes, int mode) {
 // With more than one 64^3 workgroup per CU, whole wavefronts on every SIMD count instead of one
 // workgroup's latency: 16 propagators took 27.2 us per half step with 512 threads (320: 32.8,
 // 256: 28.8) and, its registers leaving room for three workgroups of 256 threads but one of 512,
-// 53.5 us per FP64 Richardson step with 256 (320: 63.9, 512: 64.2).
+// 53.5 us per FP64 Richardson step with 256 (320: 63.9, 512: 64.2). It takes the place of a tuned shape there, unless
+// the caller has set one. Other sizes keep one shape: 32^3 and 48^3 default to 256 threads already, and larger
+// launches of 96^3 and 128^3, of 8 or 16 wavefronts a workgroup, were not tried in other shapes.
 constexpr int slab_batch_bd(int N, int mode) { return N != 64 ? 0 : (mode == SLAB_INV2 ? 256 : 512); }
 constexpr int SLAB_BATCH_BLOCKS = 256;   // workgroups of a launch above which slab_batch_bd applies: the CUs
 // kz columns: 4 in FP64 from 96^3 (the XCD tile order keeps a line's tiles on one L2)

@@ -28,7 +28,8 @@ template <typename T>
 void two_set_lds_limits() {
     static bool done = false;
     if (done) return;
-    allow_lds(&slab_two_kernel<T>);
+    allow_lds(&slab_two_kernel<T, false>);
+    if constexpr (sizeof(T) == 8) allow_lds(&slab_two_kernel<T, true>);
     allow_lds(&pencil_two_kernel<T>);
     allow_lds(&flat_steps_kernel<T, true>);
     allow_lds(&flat_steps_kernel<T, false>);
@@ -38,11 +39,21 @@ void two_set_lds_limits() {
 template <typename T>
 void Grid::launch_slab_two(int mode, const SlabBatch<T>& b, bool contiguous) const {
     // the first half step of a Richardson pair waits in the output slice
-    for (int i = 0; i < b.n; i++)
+    bool two_spectra = mode == SLAB_INV2;
+    for (int i = 0; i < b.n; i++) {
         if (mode == SLAB_INV2 && !b.it[i].qout) throw Error("slab item without the real slice its second pass reads");
+        if (mode == SLAB_FWD && b.it[i].n_out > 1) two_spectra = true;
+    }
     const TwoGeom t = two_rows(two[prec<T>()], contiguous);
-    hipLaunchKernelGGL((slab_two_kernel<T>), dim3(tnx[0], b.n), dim3(two_slab_threads(t)),
-                       two_slab_lds(t, sizeof(typename vec2<T>::type)), stream(), t, mode, b, tw<T>(1), tw<T>(2));
+    const dim3 grid(tnx[0], b.n), block(two_slab_threads(t));
+    const size_t lds = two_slab_lds(t, sizeof(typename vec2<T>::type));
+    if constexpr (sizeof(T) == 8) {
+        if (two_spectra) {
+            hipLaunchKernelGGL((slab_two_kernel<T, true>), grid, block, lds, stream(), t, mode, b, tw<T>(1), tw<T>(2));
+            return;
+        }
+    }
+    hipLaunchKernelGGL((slab_two_kernel<T, false>), grid, block, lds, stream(), t, mode, b, tw<T>(1), tw<T>(2));
 }
 
 template <typename T>

@@ -185,7 +185,12 @@ struct Emu {
         b.n = 1;
         b.it[0] = it;
         run_grid(dim3{(unsigned)n[0], 1, 1}, fts::two_slab_threads(g), fts::two_slab_lds(g, sizeof(T2)),
-                 [&] { fts::slab_two_kernel<T>(g, mode, b, tw[1].data(), tw[2].data()); });
+                 [&] {
+                     // Grid::launch_slab_two's choice
+                     if (sizeof(T) == 8 && (mode == fts::SLAB_INV2 || (mode == fts::SLAB_FWD && it.n_out > 1)))
+                         fts::slab_two_kernel<T, sizeof(T) == 8>(g, mode, b, tw[1].data(), tw[2].data());
+                     else fts::slab_two_kernel<T, false>(g, mode, b, tw[1].data(), tw[2].data());
+                 });
     }
     void pencil(T2* c, int table) {
         fts::XBatch<T> b{};
